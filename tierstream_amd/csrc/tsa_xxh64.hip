@@ -1,9 +1,8 @@
 // Device XXH64 (seed 0) for units already resident in HBM, two kernels:
 //
-//  * digest: one lane-quad per unit, lane q owns accumulator q and streams the unit's 32-byte stripes in order. XXH64
-//    keeps four dependent 64-bit chains per input, each chain a sequence of rotl(v + w*P2, 31)*P1 steps: there is no
-//    associative combine, so a unit's digest is chain-latency bound (one quad) and the kernel reaches HBM speed only
-//    with thousands of units in one launch.
+//  * digest: XXH64 keeps four dependent 64-bit chains per input, each chain a sequence of rotl(v + w*P2, 31)*P1 steps.
+//    There is no associative combine, so a unit's digest is bound by its chains: one wave runs only them, fed with the
+//    products w*P2 by four others. With very many units a quad of lanes per unit does all of it.
 //  * verify: checkpoint-parallel. The host hashes every unit once while it fills the pinned tier / the arena and keeps
 //    the four accumulators at the start of every segment (a fixed byte count inside each extent). On the device each
 //    (unit, segment) pair is an independent quad: start from the segment's checkpoint, run the segment's stripes over
@@ -124,8 +123,9 @@ __device__ __forceinline__ void init_acc(uint64_t v[4]) {
   v[3] = 0 - P1;
 }
 
-__global__ __launch_bounds__(256) void digest_kernel(const TsaUnit* __restrict__ units, uint32_t n,
-                                                     uint64_t* __restrict__ out) {
+// One unit per quad, its stripes in order by the quad itself (launches of very many units).
+__global__ __launch_bounds__(256) void digest_quads_kernel(const TsaUnit* __restrict__ units, uint32_t n,
+                                                           uint64_t* __restrict__ out) {
   const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t u = gid >> 2, q = gid & 3u;
   const bool live = u < n;
@@ -155,6 +155,242 @@ __global__ __launch_bounds__(256) void digest_kernel(const TsaUnit* __restrict__
 #pragma unroll
   for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int(base + k), 64);
   if (live && q == 0) out[u] = xfinal(all, total, tail, tail_len);
+}
+
+// ---- Whole-unit digests, one hashing wave fed by four ----
+//
+// A unit's digest is four serial chains, so a launch of few units lasts as long as its longest chain. What a round costs
+// is everything the chain's wave issues: here it is only the chain. With b = rotl(acc + w P2, 31), the accumulator is
+// b P1 and the next round is b' = rotl(b P1 + w' P2, 31): one v_mad_u64_u32 (the product's low half, w' P2 added on the
+// way), two v_mul_lo_u32, an add and two funnel shifts: 25 cycles measured for one wave, 30 with its LDS reads (61 with
+// the word's own product in the same wave). One 9 MiB unit: 11.6 -> 3.62 ms; 128 of them: 15.8 -> 3.66 ms. The products w P2 come from four other waves of the workgroup: they
+// read the units' bytes in 16-byte pieces (whole lines), multiply, and lay each chain's products next to each other in
+// LDS, so that the hashing wave takes two rounds with one ds_read_b128.
+//
+// A workgroup hashes kG units (4 kG lanes of its first wave); kG is a power of two, 512 / kG stripes of each unit make a
+// chunk (16 KiB), and three chunk buffers go round: while chunk k is hashed, chunk k+1 is complete (the hashing wave
+// reads its first stripes ahead) and the feeders write chunk k+2, with the loads of chunks k+3 and k+4 under way in
+// their registers. One barrier per chunk. The hashing wave's higher priority keeps the feeder that shares its SIMD from
+// taking its issue slots.
+constexpr uint32_t kFeeders = 256;       // feeding lanes (four waves)
+constexpr uint32_t kFeedStripes = 512;   // stripes of a chunk, all units of the workgroup
+constexpr uint32_t kFeedLoads = kFeedStripes * 2 / kFeeders;  // 16-byte pieces per lane and chunk
+constexpr uint32_t kHashAhead = 16;      // stripes the hashing wave holds in registers ahead
+
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
+typedef __attribute__((address_space(1))) const u64x2_a8 gpiece_t;
+
+constexpr uint64_t inverse64(uint64_t x) {  // modulo 2^64, x odd (Newton: each step doubles the correct bits)
+  uint64_t r = x;
+  for (int i = 0; i < 6; ++i) r *= 2 - x * r;
+  return r;
+}
+
+// A unit's stripes: stripe s lies at base[e] + 32 s for the first extent e with s < end[e].
+struct UnitStripes {
+  uintptr_t base[TSA_MAX_EXTENTS];
+  uint64_t end[TSA_MAX_EXTENTS];
+  uint64_t bytes;
+};
+
+// kHashAhead rounds on the products r, from the state b to the state b (see above). Written out because its speed hangs
+// on where the instructions lie: every one is 8 bytes long, and a lone wave issues one every 4 cycles as long as they
+// start 8-byte aligned (25 cycles a round; 31 when they straddle, as they do behind the compiler's 4-byte waits). The
+// reads of the next products stand between two such runs and cost about 5 cycles a round; spread over the rounds they
+// cost 10, and with fewer than 33 lanes active the rounds themselves are slower (31), so all lanes take part.
+#define TSA_ROUND(P)                                   \
+  "v_mad_u64_u32 v[12:13], vcc, v10, %[lo], %[" P "]\n" \
+  "v_mul_lo_u32 v14, v10, %[hi]\n"                     \
+  "v_mul_lo_u32 v15, v11, %[lo]\n"                     \
+  "v_add3_u32 v13, v15, v13, v14\n"                    \
+  "v_alignbit_b32 v11, v13, v12, 1\n"                  \
+  "v_alignbit_b32 v10, v12, v13, 1\n"
+__device__ __forceinline__ uint64_t hash_ahead(uint64_t b, const u64x2* r) {
+  uint64_t v;
+  asm volatile(
+      ".p2align 3\n"  //
+      TSA_ROUND("p0") TSA_ROUND("p1") TSA_ROUND("p2") TSA_ROUND("p3")      //
+      TSA_ROUND("p4") TSA_ROUND("p5") TSA_ROUND("p6") TSA_ROUND("p7")      //
+      TSA_ROUND("p8") TSA_ROUND("p9") TSA_ROUND("p10") TSA_ROUND("p11")    //
+      TSA_ROUND("p12") TSA_ROUND("p13") TSA_ROUND("p14") TSA_ROUND("p15")  //
+      : "={v[10:11]}"(v)
+      : "0"(b), [lo] "s"(uint32_t(P1)), [hi] "s"(uint32_t(P1 >> 32)),  //
+        [p0] "v"(r[0].x), [p1] "v"(r[0].y), [p2] "v"(r[1].x), [p3] "v"(r[1].y), [p4] "v"(r[2].x), [p5] "v"(r[2].y),
+        [p6] "v"(r[3].x), [p7] "v"(r[3].y), [p8] "v"(r[4].x), [p9] "v"(r[4].y), [p10] "v"(r[5].x), [p11] "v"(r[5].y),
+        [p12] "v"(r[6].x), [p13] "v"(r[6].y), [p14] "v"(r[7].x), [p15] "v"(r[7].y)
+      : "vcc", "v12", "v13", "v14", "v15");
+  return v;
+}
+#undef TSA_ROUND
+
+template <uint32_t kG>
+__global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit* __restrict__ units, uint32_t n,
+                                                                   uint64_t* __restrict__ out) {
+  constexpr uint32_t kC = kFeedStripes / kG;         // stripes of one unit in a chunk
+  constexpr uint32_t kRow = kC * 8 + 16;             // bytes of a chain's row (the pad spreads the rows over the banks)
+  constexpr uint32_t kBuf = 4 * kG * kRow;
+  static_assert(kC % (2 * kHashAhead) == 0, "whole register blocks per chunk");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[3 * kBuf];
+  __shared__ UnitStripes table[kG];
+  const uint32_t tid = threadIdx.x;
+  const bool feeds = tid >= 64;
+  const uint32_t mine = feeds ? (tid - 64) / (kFeeders / kG) : (tid & (4 * kG - 1)) >> 2;
+  const uint32_t u = blockIdx.x * kG + mine;
+  if (tid < kG) {
+    const uint32_t v = blockIdx.x * kG + tid;
+    const uint32_t ext = v < n ? units[v].n_ext : 0;
+    uint64_t at = 0, sum = 0;
+#pragma unroll
+    for (uint32_t e = 0; e < TSA_MAX_EXTENTS; ++e) {
+      const uint64_t bytes = e < ext ? units[v].ext[e].bytes : 0;
+      table[tid].base[e] = (e < ext ? reinterpret_cast<uintptr_t>(units[v].ext[e].ptr) : 0) - 32 * at;
+      at += bytes / 32;
+      table[tid].end[e] = at;
+      sum += bytes;
+    }
+    table[tid].bytes = sum;
+  }
+  __syncthreads();
+  const UnitStripes& us = table[mine];
+  const uint64_t total = us.end[TSA_MAX_EXTENTS - 1];
+  uint64_t most = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kG; ++i) {
+    const uint64_t t = table[i].end[TSA_MAX_EXTENTS - 1];
+    most = t > most ? t : most;
+  }
+  const uint64_t chunks = __builtin_amdgcn_readfirstlane(uint32_t((most + kC - 1) / kC >> 32)) * (1ull << 32) +
+                          __builtin_amdgcn_readfirstlane(uint32_t((most + kC - 1) / kC));
+
+  if (feeds) {
+    constexpr uint32_t kLanes = kFeeders / kG;  // of one unit: lane l moves half l & 1 of stripes l / 2 + j kLanes / 2
+    const uint32_t l = (tid - 64) % kLanes;
+    unsigned char* row = lds + (4 * mine + (l & 1u) * 2) * kRow + (l >> 1) * 8;
+    uintptr_t base = us.base[0];
+    uint64_t end = us.end[0];
+    auto load = [&](uint64_t c, u64x2* r) {
+      const uint64_t lo = c * kC;
+      if (lo >= end && lo < total)
+        for (uint32_t e = 1; e < TSA_MAX_EXTENTS && lo >= end; ++e) {
+          base = us.base[e];
+          end = us.end[e];
+        }
+      if (__all(lo + kC <= end || lo >= total)) {  // whole chunks of one extent; a unit that has ended reads its entry
+        const bool ended = lo >= total;
+        const uintptr_t p = ended ? reinterpret_cast<uintptr_t>(units) : base + 32 * (lo + (l >> 1)) + (l & 1u) * 16;
+        const uint32_t step = ended ? 0 : kLanes * 16;
+#pragma unroll
+        for (uint32_t j = 0; j < kFeedLoads; ++j) r[j] = *reinterpret_cast<gpiece_t*>(p + j * step);
+      } else {
+#pragma unroll
+        for (uint32_t j = 0; j < kFeedLoads; ++j) {
+          const uint64_t s = lo + j * (kLanes / 2) + (l >> 1);
+          uint32_t e = 0;
+          while (e + 1 < TSA_MAX_EXTENTS && s >= us.end[e]) ++e;
+          r[j] = u64x2{0, 0};
+          if (s < total) r[j] = *reinterpret_cast<gpiece_t*>(us.base[e] + 32 * s + (l & 1u) * 16);
+        }
+      }
+    };
+    auto store = [&](uint32_t b, const u64x2* r) {
+#pragma unroll
+      for (uint32_t j = 0; j < kFeedLoads; ++j) {
+        unsigned char* d = row + b * kBuf + j * (kLanes / 2) * 8;
+        *reinterpret_cast<uint64_t*>(d) = r[j].x * P2;
+        *reinterpret_cast<uint64_t*>(d + kRow) = r[j].y * P2;
+      }
+    };
+    u64x2 r0[kFeedLoads], r1[kFeedLoads];
+    load(0, r0);
+    load(1, r1);
+    store(0, r0);
+    load(2, r0);
+    store(1, r1);
+    load(3, r1);
+    __syncthreads();
+    uint32_t b = 2;
+    for (uint64_t k = 0; k < chunks; k += 2) {
+      store(b, r0);
+      load(k + 4, r0);
+      __syncthreads();
+      b = b == 2 ? 0 : b + 1;
+      if (k + 1 == chunks) break;
+      store(b, r1);
+      load(k + 5, r1);
+      __syncthreads();
+      b = b == 2 ? 0 : b + 1;
+    }
+    return;
+  }
+
+  __builtin_amdgcn_s_setprio(3);
+  const uint32_t q = tid & 3u;
+  const unsigned char* row = lds + (4 * mine + q) * kRow;
+  uint64_t acc[4];
+  init_acc(acc);
+  constexpr uint64_t kInv = inverse64(P1);
+  uint64_t b = (q == 0 ? acc[0] : q == 1 ? acc[1] : q == 2 ? acc[2] : acc[3]) * kInv;
+  auto round = [](uint64_t s, uint64_t product) { return rotl31(s * P1 + product); };
+  auto fetch = [](const unsigned char* from, u64x2* r) {
+#pragma unroll
+    for (uint32_t j = 0; j < kHashAhead / 2; ++j) r[j] = *reinterpret_cast<const u64x2*>(from + j * 16);
+  };
+  __syncthreads();
+  u64x2 a0[kHashAhead / 2], a1[kHashAhead / 2];
+  uint32_t buf = 0;
+  fetch(row, a0);
+  for (uint64_t k = 0; k < chunks; ++k) {
+    const uint32_t next = buf == 2 ? 0 : buf + 1;
+    const uint64_t done = k * kC;
+    const uint32_t left = total <= done ? 0u : total - done < kC ? uint32_t(total - done) : kC;
+    if (__all(left == 0 || left == kC)) {
+      uint64_t v = b;
+#pragma unroll 1
+      for (uint32_t s = 0; s < kC; s += 2 * kHashAhead) {
+        const bool turn = s + 2 * kHashAhead == kC;
+        const unsigned char* p = row + buf * kBuf + s * 8;
+        fetch(p + kHashAhead * 8, a1);
+        v = hash_ahead(v, a0);
+        fetch(turn ? row + next * kBuf : p + kHashAhead * 16, a0);
+        v = hash_ahead(v, a1);
+      }
+      b = left ? v : b;
+    } else {  // units that end inside this chunk: blocks that all lanes hash whole or not at all, then single stripes
+#pragma unroll 1
+      for (uint32_t s = 0; s < kC && __any(s < left); s += kHashAhead) {
+        if (__all(left <= s || left >= s + kHashAhead)) {
+          fetch(row + buf * kBuf + s * 8, a0);
+          const uint64_t v = hash_ahead(b, a0);
+          b = s < left ? v : b;
+        } else {
+#pragma unroll 1
+          for (uint32_t t = s; t < s + kHashAhead; ++t) {
+            const uint64_t v = round(b, *reinterpret_cast<const uint64_t*>(row + buf * kBuf + t * 8));
+            b = t < left ? v : b;
+          }
+        }
+      }
+      fetch(row + next * kBuf, a0);
+    }
+    buf = next;
+    __syncthreads();
+  }
+  const uint64_t v = b * P1;
+  uint64_t all[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int((tid & ~3u) + k), 64);
+  if (tid < 4 * kG && q == 0 && u < n) {
+    const uint32_t ext = units[u].n_ext < TSA_MAX_EXTENTS ? units[u].n_ext : TSA_MAX_EXTENTS;
+    const unsigned char* tail = nullptr;
+    uint32_t tail_len = 0;
+    if (ext) {
+      const uint64_t bytes = units[u].ext[ext - 1].bytes;
+      tail = static_cast<const unsigned char*>(units[u].ext[ext - 1].ptr) + bytes / 32 * 32;
+      tail_len = uint32_t(bytes % 32);
+    }
+    out[u] = xfinal(all, us.bytes, tail, tail_len);
+  }
 }
 
 // ---- The LDS-streamed check (2 KiB segments in 16-byte aligned memory) ----
@@ -516,12 +752,25 @@ __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVeri
 
 }  // namespace dev
 
+// Units per workgroup: with up to 512 one each (two workgroups on every CU), then the power of two that keeps it at 512
+// workgroups, so that every chain has a wave's full issue rate; 16 from 4097 units on, where three workgroups fit a CU's
+// LDS and 12288 units hash at once. Beyond that the workgroups would queue, and a quad per unit has lanes enough of its
+// own. Measured (us, quads / fed): 128 x 9 MiB 15847 / 3658; 512 x 1 MiB 1771 / 433; 4096 x 128 KiB 242 / 102;
+// 8192 x 64 KiB 144 / 96; 16384 x 32 KiB 112 / 130; 65536 x 8 KiB 101 / 127.
 int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipStream_t stream) {
   if (n == 0) return 0;
-  const uint32_t threads = 256;
-  const uint64_t lanes = uint64_t(n) * 4;
-  const uint32_t blocks = uint32_t((lanes + threads - 1) / threads);
-  hipLaunchKernelGGL(dev::digest_kernel, dim3(blocks), dim3(threads), 0, stream, units_dev, n, out_dev);
+  if (n > 12288) {
+    hipLaunchKernelGGL(dev::digest_quads_kernel, dim3((n + 63) / 64), dim3(256), 0, stream, units_dev, n, out_dev);
+    return int(hipGetLastError());
+  }
+  uint32_t g = 1;
+  while (g < 16 && n > 512 * g) g *= 2;
+  auto* k = g == 1   ? dev::digest_fed_kernel<1>
+            : g == 2 ? dev::digest_fed_kernel<2>
+            : g == 4 ? dev::digest_fed_kernel<4>
+            : g == 8 ? dev::digest_fed_kernel<8>
+                     : dev::digest_fed_kernel<16>;
+  hipLaunchKernelGGL(k, dim3((n + g - 1) / g), dim3(64 + dev::kFeeders), 0, stream, units_dev, n, out_dev);
   return int(hipGetLastError());
 }
 
