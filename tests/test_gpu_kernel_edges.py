@@ -57,3 +57,112 @@ def test_synth_edges(gpu, kind, words, offset):
             assert np.all(np.abs(have - want) <= np.abs(want) * 2.0 ** -8 + slack)
         else:
             assert np.array_equal(got, synth.uniform_bytes(99, 5, at, n) if kind == 0 else synth.q4_blocks(99, 5, at, n))
+
+
+# The checks by segment size and by size: all chunks of a wave in flight (1 and 2 KiB segments, up to 512 waves), two
+# chunk buffers (whole pairs of 256-byte chunks), non-temporal reads (above 80 MB), the chain loop (other segments;
+# waves with a segment that is 8-byte aligned); parts that end inside a segment, inside a stripe, or are none.
+SHAPES = [
+    (1, [2048], 2048), (1, [32], 2048), (2, [8], 2048), (1, [2080, 40], 2048), (5, [65568, 4096, 1000], 2048),
+    (64, [30 * 2048 + 32, 96], 2048), (3, [2048 * 17, 2048 * 15 + 64, 32, 2048], 2048), (3, [(8 << 20) + 32, 1 << 20], 2048),
+    (3, [28 << 20, (3 << 20) + 48], 2048), (2, [65536, 2048 + 1008], 512), (3, [65536 + 96, 1024 * 16], 1024),
+    (2, [9 << 20, 1024 * 3 + 8], 1024), (3, [1536 * 40 + 32, 1536 * 16 - 8], 1536), (2, [1 << 20, 4096 * 3 + 56], 4096),
+    (3, [28 << 20, 4096 + 16], 4096), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
+]
+
+
+def _bad_at(parts, n):
+    """A byte to spoil in each unit but the last: the first, the last, and ones next to the parts' and segments' ends."""
+    ub = sum(parts)
+    at = [0, ub - 1, parts[0] - 1, min(parts[0], ub - 1), min(2047, ub - 1), min(2048, ub - 1), max(0, parts[0] - 32), ub // 2]
+    return [at[i % len(at)] for i in range(n - 1)]
+
+
+@pytest.mark.parametrize("n,parts,seg", SHAPES)
+@pytest.mark.parametrize("staged", [False, True])
+def test_arena_checks_by_shape(gpu, n, parts, seg, staged):
+    rng = np.random.default_rng(n + sum(parts) + seg)
+    ub, slots_n = sum(parts), n + 2
+    data = rng.integers(0, 256, (n, ub), dtype=np.uint8)
+    cuts = np.cumsum([0] + parts)
+    arrays = lambda u: [u[a:b] for a, b in zip(cuts, cuts[1:])]
+    marks = [gpu.host_checkpoints(arrays(data[i]), seg) for i in range(n)]
+    keys, slots = rng.permutation(n), rng.permutation(slots_n)[:n]
+    states, digests = np.zeros((n, len(marks[0][0])), dtype=np.uint64), np.zeros(n, dtype=np.uint64)
+    for k, (st, dg) in zip(keys, marks):
+        states[k], digests[k] = st, dg
+    bufs = [gpu.DeviceBuffer(slots_n * p) for p in parts]
+    st_dev, dg_dev, fail = gpu.DeviceBuffer(states.nbytes), gpu.DeviceBuffer(digests.nbytes), gpu.DeviceBuffer(4 * n)
+    st_dev.upload(states)
+    dg_dev.upload(digests)
+    src = gpu.DeviceBuffer(n * ub)
+    a = gpu.TsaArenaVerify()
+    for p, (buf, pb) in enumerate(zip(bufs, parts)):
+        buf.upload(np.zeros(slots_n * pb, dtype=np.uint8))
+        a.arena[p], a.part_bytes[p] = buf.ptr, pb
+    a.n_parts, a.seg_bytes, a.states_dev, a.digests_dev = len(parts), seg, st_dev.ptr, dg_dev.ptr
+    for bad in ([], _bad_at(parts, n)):
+        for i, at in enumerate(bad):
+            data[i, at] ^= 0x10
+        fail.upload(np.zeros(n, dtype=np.uint32))
+        args = [C.byref(a), (C.c_uint32 * n)(*map(int, keys)), (C.c_int32 * n)(*map(int, slots)), n]
+        if staged:
+            src.upload(data.reshape(-1))
+            gpu.check(gpu.lib().tsa_xxh64_scatter_verify_slots(*args, C.c_void_p(src.ptr), C.c_void_p(fail.ptr), None))
+        else:
+            for i in range(n):
+                for buf, x in zip(bufs, arrays(data[i])):
+                    buf.upload(x, int(slots[i]) * x.nbytes)
+            gpu.check(gpu.lib().tsa_xxh64_verify_slots(*args, C.c_void_p(fail.ptr), None))
+        gpu.check(gpu.lib().tsa_stream_sync(None))
+        assert list(fail.download(4 * n).view(np.uint32)) == [1 if i < len(bad) else 0 for i in range(n)]
+        if staged:  # every unit in its slot, and nothing anywhere else
+            for p, buf in enumerate(bufs):
+                got = buf.download().reshape(slots_n, parts[p])
+                for s in range(slots_n):
+                    i = np.flatnonzero(slots == s)
+                    assert np.array_equal(got[s], arrays(data[i[0]])[p] if len(i) else np.zeros(parts[p], dtype=np.uint8))
+
+
+@pytest.mark.parametrize("align", [8, 16])
+@pytest.mark.parametrize("n,parts,seg", SHAPES + [(200, [30000 + 16, 11], 2048), (70, [32, 0], 2048), (3, [0], 2048)])
+def test_batch_checks_by_shape(gpu, n, parts, seg, align):
+    rng = np.random.default_rng(n + sum(parts) + seg + align)
+    sizes = [parts[:-1] + [parts[-1] + i % 5] for i in range(n)]
+    at, pos = 0, []
+    for unit in sizes:
+        row = []
+        for b in unit:
+            at = -(-at // align) * align + align * int(rng.integers(2))
+            row.append(at)
+            at += b
+        pos.append(row)
+    host = rng.integers(0, 256, at + 32, dtype=np.uint8)
+    buf = gpu.DeviceBuffer(host.nbytes)
+    marks = [gpu.host_checkpoints([host[p:p + b] for p, b in zip(row, unit)], seg) for row, unit in zip(pos, sizes)]
+    st_dev = gpu.DeviceBuffer(sum(st.nbytes for st, _ in marks))
+    st_dev.upload(np.concatenate([st for st, _ in marks]))
+    units, first = [], 0
+    for row, unit, (st, dg) in zip(pos, sizes, marks):
+        v = gpu.TsaVerifyUnit()
+        for e, (p, b) in enumerate(zip(row, unit)):
+            v.ext[e].ptr, v.ext[e].bytes = buf.ptr + p, b
+        v.n_ext, v.seg_first, v.states, v.digest, v.total = len(unit), first, st_dev.ptr + 32 * first, dg, sum(unit)
+        first += len(st) // 4
+        units.append(v)
+    table, fail = gpu.upload_struct_array(units), gpu.DeviceBuffer(4 * n)
+    for spoil in (False, True):
+        want = [0] * n
+        if spoil:
+            for i, o in enumerate(_bad_at(parts, n)):  # (a byte of the unit: counted through its extents)
+                for p, b in zip(pos[i], sizes[i]):
+                    if 0 <= o < b:
+                        host[p + o] ^= 0x04
+                        want[i] = 1
+                        break
+                    o -= b
+        buf.upload(host)
+        fail.upload(np.zeros(n, dtype=np.uint32))
+        gpu.check(gpu.lib().tsa_xxh64_verify(C.c_void_p(table.ptr), n, first, seg, C.c_void_p(fail.ptr), None))
+        gpu.check(gpu.lib().tsa_stream_sync(None))
+        assert list(fail.download(4 * n).view(np.uint32)) == want

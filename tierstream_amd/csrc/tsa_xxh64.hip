@@ -26,6 +26,10 @@ constexpr uint64_t P3 = 0x165667B19E3779F9ull;
 constexpr uint64_t P4 = 0x85EBCA77C2B2AE63ull;
 constexpr uint64_t P5 = 0x27D4EB2F165667C5ull;
 
+typedef __attribute__((address_space(1))) const uint64_t gword_t;
+typedef __attribute__((address_space(1))) uint64_t gout_t;
+typedef __attribute__((address_space(1))) const unsigned char gbyte_t;
+
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int r) { return (x << r) | (x >> (64 - r)); }
 // rotl by 31 as two funnel shifts (v_alignbit_b32) on the 32-bit halves: hi' = (hi:lo) >> 1, lo' = (lo:hi) >> 1
 __device__ __forceinline__ uint64_t rotl31(uint64_t x) {
@@ -33,10 +37,47 @@ __device__ __forceinline__ uint64_t rotl31(uint64_t x) {
   return uint64_t(__builtin_amdgcn_alignbit(hi, lo, 1u)) << 32 | __builtin_amdgcn_alignbit(lo, hi, 1u);
 }
 __device__ __forceinline__ uint64_t xround(uint64_t acc, uint64_t w) { return rotl31(acc + w * P2) * P1; }
+// The same round on the state b = acc * P1^-1 (mod 2^64): b' = rotl(b * P1 + w * P2, 31), where the sum costs nothing
+// (v_mad_u64_u32 adds the product on the way).
+constexpr uint64_t inverse64(uint64_t x) {  // modulo 2^64, x odd (Newton: each step doubles the correct bits)
+  uint64_t r = x;
+  for (int i = 0; i < 6; ++i) r *= 2 - x * r;
+  return r;
+}
+constexpr uint64_t P1inv = inverse64(P1);
+__device__ __forceinline__ uint64_t bround(uint64_t b, uint64_t product) { return rotl31(b * P1 + product); }
 __device__ __forceinline__ uint64_t xmerge(uint64_t h, uint64_t v) { return (h ^ xround(0, v)) * P1 + P4; }
 
-// Digest of the four accumulators, the total length and the (< 32 byte) tail. Runs on one lane.
-__device__ uint64_t xfinal(const uint64_t v[4], uint64_t total, const unsigned char* tail, uint32_t tail_len) {
+// A unit's last (< 32) bytes in registers: whole words, then the rest (p is 8-byte aligned).
+struct Tail {
+  uint64_t word[3] = {0, 0, 0};
+  uint64_t rest = 0;
+  uint32_t len = 0;
+};
+__device__ __forceinline__ Tail load_tail(const unsigned char* p, uint32_t len) {
+  Tail t;
+  t.len = len;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+#pragma unroll
+  for (uint32_t i = 0; i < 3; ++i)
+    if (8 * i + 8 <= len) t.word[i] = *reinterpret_cast<gword_t*>(at + 8 * i);
+  if (const uint32_t n = len & 7u) {  // (all its bytes at once: one after the other, each was a memory latency)
+#pragma unroll
+    for (uint32_t b = 0; b < 7; ++b)
+      t.rest |= uint64_t(*reinterpret_cast<gbyte_t*>(at + (len & ~7u) + (b < n ? b : n - 1))) << (8 * b);
+    t.rest &= (1ull << (8 * n)) - 1;
+  }
+  return t;
+}
+__device__ __forceinline__ void store_tail(unsigned char* p, const Tail& t) {
+#pragma unroll
+  for (uint32_t i = 0; i < 3; ++i)
+    if (8 * i + 8 <= t.len) *reinterpret_cast<uint64_t*>(p + 8 * i) = t.word[i];
+  for (uint32_t b = t.len & ~7u; b < t.len; ++b) p[b] = static_cast<unsigned char>(t.rest >> (8 * (b & 7u)));
+}
+
+// Digest of the four accumulators, the total length and the tail. Runs on one lane.
+__device__ __forceinline__ uint64_t xfinal(const uint64_t v[4], uint64_t total, const Tail& t) {
   uint64_t h;
   if (total >= 32) {
     h = rotl64(v[0], 1) + rotl64(v[1], 7) + rotl64(v[2], 12) + rotl64(v[3], 18);
@@ -45,22 +86,22 @@ __device__ uint64_t xfinal(const uint64_t v[4], uint64_t total, const unsigned c
     h = P5;  // seed 0
   }
   h += total;
-  uint32_t i = 0;
-  for (; i + 8 <= tail_len; i += 8) {
-    uint64_t w = 0;
-    for (int b = 7; b >= 0; --b) w = (w << 8) | tail[i + b];
-    h ^= xround(0, w);
-    h = rotl64(h, 27) * P1 + P4;
-  }
-  if (i + 4 <= tail_len) {
-    const uint32_t w = uint32_t(tail[i]) | uint32_t(tail[i + 1]) << 8 | uint32_t(tail[i + 2]) << 16 |
-                       uint32_t(tail[i + 3]) << 24;
-    h ^= uint64_t(w) * P1;
+#pragma unroll
+  for (uint32_t i = 0; i < 3; ++i)
+    if (8 * i + 8 <= t.len) {
+      h ^= xround(0, t.word[i]);
+      h = rotl64(h, 27) * P1 + P4;
+    }
+  uint64_t rest = t.rest;
+  uint32_t n = t.len & 7u;
+  if (n >= 4) {
+    h ^= (rest & 0xFFFFFFFFull) * P1;
     h = rotl64(h, 23) * P2 + P3;
-    i += 4;
+    rest >>= 32;
+    n -= 4;
   }
-  for (; i < tail_len; ++i) {
-    h ^= uint64_t(tail[i]) * P5;
+  for (; n > 0; --n, rest >>= 8) {
+    h ^= (rest & 0xFFu) * P5;
     h = rotl64(h, 11) * P1;
   }
   h ^= h >> 33;
@@ -81,10 +122,9 @@ __device__ uint64_t xfinal(const uint64_t v[4], uint64_t total, const unsigned c
 // Measured on one 336 MiB unit (8 KiB segments): this loop reads at 5.8 TB/s, 95 % of what a fully coalesced 16-byte
 // streaming read of the same bytes reaches in one launch (6.1 TB/s); the rounds alone (no loads) run at 17 TB/s. So
 // the kernel is bound by the read, not the multiplies, and neither a software-pipelined nor an LDS-staged variant
-// (coalesced 16-byte loads into LDS, chains run from LDS) beat it.
+// (coalesced 16-byte loads into LDS, chains run from LDS) beat it. Sixteen stripes a block: with 32 or 64 in registers
+// (one or two memory latencies a segment) 25 MB of 8-byte aligned units took 8.2 and 9.5 us against 7.6.
 constexpr int kBlock = 16;
-typedef __attribute__((address_space(1))) const uint64_t gword_t;
-typedef __attribute__((address_space(1))) uint64_t gout_t;
 
 // kCopy: each word read is also stored at the same offset from d (the staged unit's bytes into their arena slot while
 // they are hashed: the bytes cross HBM once each way).
@@ -154,7 +194,7 @@ __global__ __launch_bounds__(256) void digest_quads_kernel(const TsaUnit* __rest
   const uint32_t base = threadIdx.x & ~3u;
 #pragma unroll
   for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int(base + k), 64);
-  if (live && q == 0) out[u] = xfinal(all, total, tail, tail_len);
+  if (live && q == 0) out[u] = xfinal(all, total, load_tail(tail, tail_len));
 }
 
 // ---- Whole-unit digests, one hashing wave fed by four ----
@@ -180,12 +220,6 @@ constexpr uint32_t kHashAhead = 16;      // stripes the hashing wave holds in re
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
 typedef __attribute__((address_space(1))) const u64x2_a8 gpiece_t;
-
-constexpr uint64_t inverse64(uint64_t x) {  // modulo 2^64, x odd (Newton: each step doubles the correct bits)
-  uint64_t r = x;
-  for (int i = 0; i < 6; ++i) r *= 2 - x * r;
-  return r;
-}
 
 // A unit's stripes: stripe s lies at base[e] + 32 s for the first extent e with s < end[e].
 struct UnitStripes {
@@ -329,9 +363,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
   const unsigned char* row = lds + (4 * mine + q) * kRow;
   uint64_t acc[4];
   init_acc(acc);
-  constexpr uint64_t kInv = inverse64(P1);
-  uint64_t b = (q == 0 ? acc[0] : q == 1 ? acc[1] : q == 2 ? acc[2] : acc[3]) * kInv;
-  auto round = [](uint64_t s, uint64_t product) { return rotl31(s * P1 + product); };
+  uint64_t b = (q == 0 ? acc[0] : q == 1 ? acc[1] : q == 2 ? acc[2] : acc[3]) * P1inv;
   auto fetch = [](const unsigned char* from, u64x2* r) {
 #pragma unroll
     for (uint32_t j = 0; j < kHashAhead / 2; ++j) r[j] = *reinterpret_cast<const u64x2*>(from + j * 16);
@@ -366,7 +398,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
         } else {
 #pragma unroll 1
           for (uint32_t t = s; t < s + kHashAhead; ++t) {
-            const uint64_t v = round(b, *reinterpret_cast<const uint64_t*>(row + buf * kBuf + t * 8));
+            const uint64_t v = bround(b, *reinterpret_cast<const uint64_t*>(row + buf * kBuf + t * 8));
             b = t < left ? v : b;
           }
         }
@@ -389,263 +421,429 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
       tail = static_cast<const unsigned char*>(units[u].ext[ext - 1].ptr) + bytes / 32 * 32;
       tail_len = uint32_t(bytes % 32);
     }
-    out[u] = xfinal(all, us.bytes, tail, tail_len);
+    out[u] = xfinal(all, us.bytes, load_tail(tail, tail_len));
   }
 }
 
-// ---- The LDS-streamed check (2 KiB segments in 16-byte aligned memory) ----
+// ---- The LDS-streamed check (segments of a multiple of 512 bytes) ----
 //
 // The chain loop above reads 8 bytes per lane at a 32-byte stride: every load instruction of a wave touches 16 lines
 // (one per quad) and relies on the CU cache to keep each line for the next three. Here every wave streams its 16
 // segments through LDS instead, with direct-to-LDS 16-byte loads (global_load_lds_dwordx4): 64 lanes fill 1 KiB of
-// LDS per instruction, eight whole 128-byte lines, with the non-temporal hint (the bytes are read once). The quads
-// then run their chains from LDS. Measured on one 336 MiB unit: 52-53 us against 58 us for the chain loop, the same
-// as a plain coalesced 16-byte streaming read of the unit.
+// LDS per instruction, eight whole 128-byte lines. The quads then run their chains from LDS. Only for waves whose
+// segments are 16-byte aligned: pieces that straddle two lines' halves made 34 MB of 8-byte aligned units 12.1 us, the
+// chain loop 10.7.
 //
 // Per wave: a chunk is 256 bytes (8 stripes) of each of its 16 segments, 4 KiB, four loads: load k carries segments
 // 4k..4k+3, lanes 16i..16i+15 the 16 pieces of segment 4k+i. A segment's stripes are rotated by (its quad index mod 8)
 // inside its 256 bytes, so that the wave's ds_read_b64 of one stripe of all 16 segments spreads over the LDS banks.
-// Two chunk buffers per wave: the loads of chunk c+2 are issued when chunk c has been hashed. The loads are inline
-// assembly, so the compiler neither waits for them nor knows them; each chunk waits for its own loads with an explicit
-// vmcnt (loads complete in order) and the buffer is reused only after its LDS reads have completed (lgkmcnt 0).
-// Lanes whose piece lies past their segment's stripes load the segment's first bytes instead (never out of bounds),
-// and every wave issues the same number of loads, which the vmcnt counts rely on.
-constexpr uint32_t kLdsSegBytes = 2048;  // 8 chunks of 256 bytes per segment
-constexpr uint32_t kLdsChunks = kLdsSegBytes / 256;
-constexpr uint32_t kLdsWaveBytes = 2 * 4096;  // two chunk buffers
+// Before the chunks goes one load of every quad's checkpoint and the one after it (64 contiguous bytes): read where it
+// is used, the checkpoint held every chunk's loads back, and the next one cost a memory latency at the end.
+// The loads are inline assembly, so the compiler neither waits for them nor knows them; each chunk waits for its own
+// loads with an explicit vmcnt (loads complete in order, and a load or store of the compiler's among them only makes
+// the wait longer). Lanes whose piece lies past their segment's stripes load an earlier piece again (never out of
+// bounds), and every wave issues the same number of loads, which the vmcnt counts rely on. The instruction's offset
+// moves both addresses, so the chunks of a wave of whole segments take no address arithmetic. A chunk that every
+// segment has whole or not at all is hashed without a select per round: waves at the end of a part are as fast as the
+// others (with both costs in them they were the launch's last: 8 MB in 5.5 us instead of 6.3).
+//
+// What bounds it: reading, from about 50 MB on (336 MiB 55 us, 6.5 TB/s); below, one launch and one to four memory
+// latencies (192 KiB 4.8 us, of which a launch of nothing takes 3.7).
+constexpr uint32_t kStateBytes = 1024;  // per wave, at the end of its LDS: 64 bytes per quad
 
-__device__ __forceinline__ void lds_load16(const unsigned char* g, uint32_t lds_addr) {
-  uint32_t save;  // M0 (the LDS destination) is restored for the compiler; s_nop: an M0 write before an LDS load
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off nt\n\t"
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0"
-      : "=&s"(save)
-      : "v"(g), "s"(lds_addr)
-      : "memory");
-}
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) u32x4 gu32x4_t;
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+typedef __attribute__((address_space(1))) u32x4_a8 gu32x4_t;
+
+// M0 (the LDS destination) is restored for the compiler; s_nop: an M0 write before a load to LDS.
+#define TSA_LDS_LOAD16(HINT)                         \
+  asm volatile(                                      \
+      "s_mov_b32 %0, m0\n\t"                         \
+      "s_mov_b32 m0, %2\n\t"                         \
+      "s_nop 0\n\t"                                  \
+      "global_load_lds_dwordx4 %1, off" HINT "\n\t"  \
+      "s_mov_b32 m0, %0\n\t"                         \
+      "s_nop 0"                                      \
+      : "=&s"(save)                                  \
+      : "v"(g), "s"(lds_addr)                        \
+      : "memory")
+template <bool kNt>
+__device__ __forceinline__ void lds_load16(const unsigned char* g, uint32_t lds_addr) {
+  uint32_t save;
+  if constexpr (kNt)
+    TSA_LDS_LOAD16(" nt");
+  else
+    TSA_LDS_LOAD16("");
+}
+#undef TSA_LDS_LOAD16
+// A chunk of whole segments: piece k of the lane at g[k] + kAt to lds_addr + 1024 k.
+#define TSA_LDS_LOAD_CHUNK(HINT)                                                                       \
+  asm volatile(                                                                                        \
+      "s_mov_b32 %0, m0\n\t"                                                                           \
+      "s_mov_b32 m0, %5\n\t"                                                                           \
+      "s_nop 0\n\t"                                                                                    \
+      "global_load_lds_dwordx4 %1, off offset:%6" HINT "\n\t"                                          \
+      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
+      "s_nop 0\n\t"                                                                                    \
+      "global_load_lds_dwordx4 %2, off offset:%6" HINT "\n\t"                                          \
+      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
+      "s_nop 0\n\t"                                                                                    \
+      "global_load_lds_dwordx4 %3, off offset:%6" HINT "\n\t"                                          \
+      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
+      "s_nop 0\n\t"                                                                                    \
+      "global_load_lds_dwordx4 %4, off offset:%6" HINT "\n\t"                                          \
+      "s_mov_b32 m0, %0\n\t"                                                                           \
+      "s_nop 0"                                                                                        \
+      : "=&s"(save)                                                                                    \
+      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr - kAt), "n"(kAt)                      \
+      : "memory", "scc")
+template <uint32_t kAt, bool kNt>
+__device__ __forceinline__ void lds_load_chunk(const unsigned char* const g[4], uint32_t lds_addr) {
+  uint32_t save;
+  if constexpr (kNt)
+    TSA_LDS_LOAD_CHUNK(" nt");
+  else
+    TSA_LDS_LOAD_CHUNK("");
+}
+#undef TSA_LDS_LOAD_CHUNK
 
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// The wave's 16 quads (lane = 4 j + q) each hash `stripes` (<= 64) stripes from `from` (16-byte aligned) starting at
-// state v; all 64 lanes must call it. lds: the wave's kLdsWaveBytes of LDS (its address and its 32-bit LDS offset).
-// kCopy: every stripe is also written to the same offset from `to` (16-byte aligned), each lane storing the 16-byte
-// pieces it loaded, from LDS, once they have landed.
-template <bool kCopy>
-__device__ __forceinline__ uint64_t lds_chain_t(uint64_t v, const unsigned char* from, unsigned char* to,
-                                                uint32_t stripes, const unsigned char* lds, uint32_t lds_off) {
+// A wave's part of its workgroup's LDS: its address and its 32-bit LDS address.
+struct WaveLds {
+  unsigned char* p;
+  uint32_t off;
+};
+__device__ __forceinline__ WaveLds wave_lds(unsigned char* lds, uint32_t bytes) {
+  unsigned char* p = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * bytes;
+  return {p, uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(p)))};
+}
+
+template <uint32_t kD, bool kNt, uint32_t kC = 0>
+__device__ __forceinline__ void issue_all(const unsigned char* const g[4], uint32_t lds_off) {
+  if constexpr (kC < kD) {
+    lds_load_chunk<kC * 256, kNt>(g, lds_off + kC * 4096);
+    issue_all<kD, kNt, kC + 1>(g, lds_off);
+  }
+}
+// Chunk by chunk, each when it has landed (the later ones' loads may still be in flight).
+template <uint32_t kD, uint32_t kC = 0, class F>
+__device__ __forceinline__ void drain(F&& hash) {
+  if constexpr (kC < kD) {
+    wait_loads<4 * (kD - 1 - kC)>();
+    hash(kC);
+    drain<kD, kC + 1>(hash);
+  }
+}
+
+// One wave's 16 segments (quad j's lanes 4 j + q hold segment j): where it is read and (kCopy) written, its stripes (0
+// hashes nothing and reads 16 bytes), its checkpoint (32 bytes, 64 when it is not the unit's last). Out: the
+// accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
+// go along with the first live segment and their results mean nothing. The wave's LDS has lds_bytes<kD>().
+//
+// kD = 2: two chunk buffers, chunk c+2 loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0). kD > 2:
+// segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy, whose stores
+// the waits would wait for).
+template <uint32_t kD>
+constexpr uint32_t lds_bytes() {
+  return kD * 4096 + kStateBytes;
+}
+template <uint32_t kD, bool kNt, bool kCopy>
+__device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
+                                              uint32_t stripes, const uint64_t* state, bool last,
+                                              const WaveLds& w, uint64_t* next) {
+  const unsigned char* lds = w.p;
+  const uint32_t lds_off = w.off;
   const uint32_t lane = threadIdx.x & 63u, q = lane & 3u, j = lane >> 2;
   const uint32_t i = lane >> 4, m = lane & 15u;
+  const int first = __ffsll(static_cast<long long>(__ballot(live))) - 1;
+  auto from_first = [&](uint64_t x, uint64_t mine) {
+    const uint64_t f = __shfl(static_cast<unsigned long long>(x), first, 64);
+    return live ? mine : f;
+  };
+  from = reinterpret_cast<const unsigned char*>(from_first(reinterpret_cast<uintptr_t>(from), reinterpret_cast<uintptr_t>(from)));
+  state = reinterpret_cast<const uint64_t*>(from_first(reinterpret_cast<uintptr_t>(state), reinterpret_cast<uintptr_t>(state)));
+  last = last || !live;
+  static_assert(kD == 2 || !kCopy, "");
+  uint32_t chunks = kD;
+  if (kD == 2) {  // as many pairs as the wave's longest segment has
+    uint32_t most = stripes;
+#pragma unroll
+    for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
+    chunks = max(2u, __builtin_amdgcn_readfirstlane((most + 15) / 16 * 2));
+  }
+  const bool whole = __all(!live || stripes == 8 * chunks);
+  lds_load16<kNt>(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
+  // The lane's piece of load k (of segment 4k + i: quad 4k + i's lane 0 holds its source) in chunk 0, and how far its
+  // segment has later ones: past that the lane loads the last one again, or (no stripe of its own) the segment's first.
   const unsigned char* src[4];
   unsigned char* dst[4];
-  uint32_t n[4];
+  uint32_t n[4], g0[4], lim[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {  // the lane loads for segment 4k + i (quad 4k + i's lane 0 holds its source)
+  for (int k = 0; k < 4; ++k) {
     const int owner = int((4 * k + i) * 4);
+    g0[k] = ((m >> 1) - ((4 * k + i) & 7u)) & 7u;  // its stripe in chunk 0
+    n[k] = uint32_t(__shfl(int(stripes), owner, 64));
+    const uint32_t at = g0[k] * 32 + (m & 1u) * 16;
     src[k] = reinterpret_cast<const unsigned char*>(
-        __shfl(static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(from)), owner, 64));
+                 __shfl(static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(from)), owner, 64)) +
+             (whole || g0[k] < n[k] ? at : 0);
+    lim[k] = g0[k] < n[k] ? (n[k] - 1 - g0[k]) / 8 * 256 : 0;
     if (kCopy)
       dst[k] = reinterpret_cast<unsigned char*>(
-          __shfl(static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(to)), owner, 64));
-    n[k] = uint32_t(__shfl(int(stripes), owner, 64));
+                   __shfl(static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(to)), owner, 64)) +
+               at;
   }
-  auto piece = [&](uint32_t c, uint32_t k) {  // the global stripe this lane's piece of load k of chunk c holds
-    return (((m >> 1) - ((4 * k + i) & 7u)) & 7u) + 8 * c;
-  };
-  auto issue = [&](uint32_t c) {
+  auto issue_part = [&](uint32_t c, uint32_t buf) {  // not only whole segments
+    const unsigned char* g[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-      const uint32_t g = piece(c, k);
-      const unsigned char* at = g < n[k] ? src[k] + g * 32 + (m & 1u) * 16 : src[k];
-      lds_load16(at, lds_off + (c & 1u) * 4096 + k * 1024);
+    for (uint32_t k = 0; k < 4; ++k) g[k] = src[k] + min(256 * c, lim[k]);
+    lds_load_chunk<0, kNt>(g, lds_off + buf * 4096);
+  };
+  const bool full = kCopy && __all(live && stripes == 8 * chunks);
+  auto store = [&](uint32_t c, uint32_t buf) {  // the lane's own four pieces, as they landed in LDS
+    u32x4 x[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const u32x4*>(lds + buf * 4096 + k * 1024 + lane * 16);
+    // (global stores: a generic one would also count on the LDS counter)
+    if (full) {
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(dst[k] + c * 256)) = x[k];
+    } else {
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k)
+        if (g0[k] + 8 * c < n[k]) *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(dst[k] + c * 256)) = x[k];
     }
   };
-  issue(0);
-  issue(1);
-  // v (the segment's checkpoint) arrives here: the compiler's wait for it (a vmcnt(0), which also covers the two
-  // chunks just issued) then sits before the loop, not inside it at every use of the loop-carried state
-  asm volatile("" : "+v"(v));
   const uint32_t rot = j & 7u;
   const unsigned char* rd = lds + (j >> 2) * 1024 + (j & 3u) * 256 + q * 8;
-  auto hash = [&](uint32_t c) {
-    if (kCopy) {  // the lane's own four pieces, as they landed in LDS
+  uint64_t b = 0;
+  auto hash = [&](uint32_t c, uint32_t buf) {
+    uint64_t x[8];
 #pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t g = piece(c, k);
-        const u32x4 x = *reinterpret_cast<const u32x4*>(lds + (c & 1u) * 4096 + k * 1024 + lane * 16);
-        if (g < n[k])  // (a global store: a generic one would also count on the LDS counter waited on below)
-          *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(dst[k] + g * 32 + (m & 1u) * 16)) = x;
+    for (uint32_t t = 0; t < 8; ++t)
+      x[t] = *reinterpret_cast<const uint64_t*>(rd + ((t + rot) & 7u) * 32 + buf * 4096);
+    const bool in = 8 * c < stripes;
+    if (whole || __all(!in || stripes >= 8 * c + 8)) {  // every segment has all of the chunk or none of it
+      uint64_t r = b;
+#pragma unroll
+      for (uint32_t t = 0; t < 8; ++t) r = bround(r, x[t] * P2);
+      b = whole || in ? r : b;
+    } else {
+#pragma unroll
+      for (uint32_t t = 0; t < 8; ++t) {
+        uint64_t r = bround(b, x[t] * P2);
+        asm volatile("" : "+v"(r));  // (a select, not a branch around each round)
+        b = 8 * c + t < stripes ? r : b;
       }
     }
-    const unsigned char* b = rd + (c & 1u) * 4096;
-#pragma unroll
-    for (uint32_t t = 0; t < 8; ++t) {
-      const uint64_t x = *reinterpret_cast<const uint64_t*>(b + ((t + rot) & 7u) * 32);
-      const uint64_t r = xround(v, x);
-      v = 8 * c + t < stripes ? r : v;
-    }
   };
-  // chunks 0 .. kLdsChunks - 3: the next chunk's four loads may still be in flight (vmcnt 4 also holds with the copy's
-  // stores among them: loads complete in order among themselves); then this buffer is refilled
-#pragma unroll 2
-  for (uint32_t c = 0; c + 2 < kLdsChunks; ++c) {
+  auto states = [&] {
+    const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kD * 4096 + j * 64);
+    b = st[q] * P1inv;
+    *next = st[4 + q];
+  };
+  if constexpr (kD == 2) {
+    auto issue = [&](uint32_t c, uint32_t buf) {
+      if (whole) {
+        lds_load_chunk<0, kNt>(src, lds_off + buf * 4096);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) src[k] += 256;
+      } else {
+        issue_part(c, buf);
+      }
+    };
+    issue(0, 0);
+    issue(1, 1);
+    wait_loads<8>();
+    states();
+    for (uint32_t c = 0; c + 2 < chunks; c += 2) {
+      wait_loads<4>();
+      if (kCopy) store(c, 0);
+      hash(c, 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue(c + 2, 0);
+      wait_loads<4>();
+      if (kCopy) store(c + 1, 1);
+      hash(c + 1, 1);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue(c + 3, 1);
+    }
     wait_loads<4>();
-    hash(c);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this buffer's LDS reads are done before it is refilled
-    issue(c + 2);
+    if (kCopy) store(chunks - 2, 0);
+    hash(chunks - 2, 0);
+    wait_loads<0>();
+    if (kCopy) store(chunks - 1, 1);
+    hash(chunks - 1, 1);
+  } else {
+    if (whole) {
+      issue_all<kD, kNt>(src, lds_off);
+    } else {
+#pragma unroll 1
+      for (uint32_t c = 0; c < kD; ++c) issue_part(c, c);
+    }
+    wait_loads<4 * kD>();
+    states();
+    drain<kD>([&](uint32_t c) { hash(c, c); });
   }
-  wait_loads<4>();
-  hash(kLdsChunks - 2);
-  wait_loads<0>();
-  hash(kLdsChunks - 1);
-  return v;
-}
-__device__ __forceinline__ uint64_t lds_chain(uint64_t v, const unsigned char* from, uint32_t stripes,
-                                              const unsigned char* lds, uint32_t lds_off) {
-  return lds_chain_t<false>(v, from, nullptr, stripes, lds, lds_off);
+  return b * P1;
 }
 
 // The chain-loop kernels (dg_verify_kernel, dg_scatter_verify_kernel) are held to 8 waves per SIMD (at most 64
 // VGPRs): unbounded, the compiler spends registers on scheduling (83-86 VGPRs, 5 waves per SIMD) and the kernel has
 // 5/8 of the loads in flight it could; bounded it needs 52-58 with no spill, and one 336 MiB unit's check (3 parts,
 // 2 KiB segments, timed alone in a fresh process) ran 67 -> 62 us. The LDS-streamed kernels keep their loads in LDS,
-// not in registers, and run 5 waves per SIMD (their 32 KiB of LDS per workgroup).
+// not in registers.
 #define TSA_VERIFY_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
 
-// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). A wave
-// whose segments are all 2 KiB pieces of 16-byte aligned extents, each of at least one stripe, streams them through
-// LDS (lds_chain); any other wave (other segment sizes, unaligned extents, a last extent under 32 bytes) runs the
-// chain loop. The choice is the wave's: all its lanes take one path.
-__global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
-                                                     uint64_t n_segments, uint64_t seg_bytes,
-                                                     uint32_t* __restrict__ fail) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kLdsWaveBytes];
-  const uint64_t gid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const uint64_t s = gid >> 2;
-  const uint32_t q = uint32_t(gid & 3u);
-  bool live = s < n_segments;
-  uint32_t ui = 0;
-  if (live) {  // the unit holding global segment s (units sorted by seg_first)
-    uint32_t lo = 0, hi = n_units;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) / 2;
-      if (units[mid].seg_first <= s) lo = mid;
-      else hi = mid;
-    }
-    ui = lo;
+// The last unit of [0, n_units) whose seg_first is at most s (ascending): 64 probes at a time.
+__device__ __forceinline__ uint32_t unit_of(const TsaVerifyUnit* units, uint32_t n_units, uint64_t s) {
+  uint32_t lo = 0, hi = n_units;
+  while (hi - lo > 1) {
+    const uint32_t step = (hi - lo + 63) / 64, at = lo + (threadIdx.x & 63u) * step;
+    const bool under = at < hi && at >= lo && units[at].seg_first <= s;
+    const uint32_t k = uint32_t(__popcll(__ballot(under)));
+    lo += (k ? k - 1 : 0) * step;
+    hi = hi - lo < step ? hi : lo + step;
   }
-  uint64_t v = 0;
-  bool last = false;
-  uint64_t local = 0, total = 0, stripes = 0;
+  return lo;
+}
+
+// A segment of a unit given by its extents: where it lies and what it must lead to.
+struct HostSeg {
   const unsigned char* from = nullptr;
+  const uint64_t* state = nullptr;
+  uint64_t digest = 0, total = 0;
+  uint32_t stripes = 0, ui = 0;
+  bool live = false, last = false;
+  Tail tail;
+};
+// shift: seg_bytes = 1 << shift, or 64 when it is no power of two (a 64-bit division is about 100 instructions).
+__device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_t ui, uint64_t s, uint64_t seg_bytes,
+                                                uint32_t shift, uint32_t* fail, uint32_t q) {
+  HostSeg g;
+  g.ui = ui;
+  const uint64_t local = s - un.seg_first;  // the unit's segment index (its checkpoint index)
+  const uint32_t n_ext = un.n_ext;
+  uint64_t k = local;
+  bool found = false;
   const unsigned char* tail = nullptr;
   uint32_t tail_len = 0;
-  const TsaVerifyUnit* un = units + ui;
-  if (live) {
-    local = s - un->seg_first;  // the unit's segment index (its checkpoint index)
-    // the extent and the segment inside it
-    uint64_t k = local;
-    uint32_t e = 0;
-    for (; e < un->n_ext; ++e) {
-      const uint64_t b = un->ext[e].bytes;
-      const bool last_ext = e + 1 == un->n_ext;
+#pragma unroll
+  for (uint32_t e = 0; e < TSA_MAX_EXTENTS; ++e) {
+    if (e < n_ext && !found) {
+      const uint64_t b = un.ext[e].bytes;
+      const bool last_ext = e + 1 == n_ext;
       const uint64_t span = last_ext ? b / 32 * 32 : b;
-      uint64_t nseg = (span + seg_bytes - 1) / seg_bytes;
+      uint64_t nseg = shift < 64 ? (span + seg_bytes - 1) >> shift : (span + seg_bytes - 1) / seg_bytes;
       if (last_ext && nseg == 0) nseg = 1;
       if (k < nseg) {
+        found = true;
+        const unsigned char* p = static_cast<const unsigned char*>(un.ext[e].ptr);
         const uint64_t off = k * seg_bytes;
         const uint64_t end = off + seg_bytes < span ? off + seg_bytes : span;
-        stripes = (end - off) / 32;
-        from = static_cast<const unsigned char*>(un->ext[e].ptr) + off;
-        last = last_ext && k + 1 == nseg;
-        if (last) {
-          tail = static_cast<const unsigned char*>(un->ext[e].ptr) + span;
-          tail_len = uint32_t(b - span);
-        }
-        break;
+        g.stripes = uint32_t((end - off) / 32);
+        g.from = p + off;
+        g.last = last_ext && k + 1 == nseg;
+        tail = p + span;
+        tail_len = uint32_t(b - span);
       }
       k -= nseg;
     }
-    if (e == un->n_ext) {  // the launch's prefix sums disagree with the extents: reported, nothing read or checked
-      if (q == 0) atomicOr(fail + ui, 2u);
-      live = false;
-    } else {
-      v = un->states[4 * local + q];
-      total = un->total;
-    }
   }
-  const uint64_t lanes_live = __ballot(live);
-  if (lanes_live == 0) return;  // (the whole wave)
-  const bool lds_path = seg_bytes == kLdsSegBytes &&
-                        __all(!live || ((reinterpret_cast<uintptr_t>(from) & 15u) == 0 && stripes >= 1));
-  if (lds_path) {
-    // a dead lane streams a live lane's segment (in bounds) and hashes none of it
-    const unsigned char* any = reinterpret_cast<const unsigned char*>(__shfl(
-        static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(from)), __ffsll((long long)lanes_live) - 1, 64));
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned char* mine = lds + wave * kLdsWaveBytes;
-    const uint32_t mine_off =
-        uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(mine)));
-    v = lds_chain(v, live ? from : any, live ? uint32_t(stripes) : 0u, mine, mine_off);
-  } else if (live) {
-    v = chain(v, from, stripes, q);
+  if (!found) {  // the launch's prefix sums disagree with the extents: reported, nothing read or checked
+    if (q == 0) atomicOr(fail + ui, 2u);
+    return g;
+  }
+  if (g.last && q == 0) g.tail = load_tail(tail, tail_len);
+  g.live = true;
+  g.state = un.states + 4 * local;
+  g.digest = un.digest;
+  g.total = un.total;
+  return g;
+}
+// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
+// lds_check; 0 runs the chain loop from memory.
+template <uint32_t kD, bool kNt, uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
+                                                          uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
+                                                          uint32_t* __restrict__ fail) {
+  const uint64_t s0 = (uint64_t(blockIdx.x) * kThreads + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u)) >> 2;
+  if (s0 >= n_segments) return;  // (the whole wave)
+  const uint32_t q = threadIdx.x & 3u;
+  const uint64_t s = s0 + ((threadIdx.x & 63u) >> 2);
+  const uint64_t end = n_segments - s0 < 16 ? n_segments : s0 + 16;
+  uint32_t ui = unit_of(units, n_units, s0);
+  HostSeg g;
+  const uint64_t after = ui + 1 < n_units ? units[ui + 1].seg_first : ~0ull;
+  const TsaVerifyUnit un = units[ui];  // (whole and at once: with scalar loads, one memory latency)
+  if (after >= end) {
+    if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
+  } else if (s < end) {
+    while (ui + 1 < n_units && units[ui + 1].seg_first <= s) ++ui;
+    const TsaVerifyUnit mine = units[ui];
+    g = host_segment(mine, ui, s, seg_bytes, shift, fail, q);
+  }
+  if (__ballot(g.live) == 0) return;
+  uint64_t v = 0, next = 0;
+  bool streamed = false;
+  if constexpr (kD != 0) {
+    streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kThreads / 64 * lds_bytes<kD>()];
+    if (streamed)
+      v = lds_check<kD, kNt, false>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr,
+                                    g.stripes, g.state, g.last, wave_lds(lds, lds_bytes<kD>()), &next);
+  }
+  if (!streamed && g.live) {
+    next = g.last ? 0 : g.state[4 + q];
+    v = chain_t<false>(g.state[q], g.from, nullptr, g.stripes, q);
   }
   uint64_t all[4];
   const uint32_t base = threadIdx.x & ~3u;
 #pragma unroll
   for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int(base + k), 64);
-  if (!live) return;
-  if (!last) {
-    if (v != un->states[4 * (local + 1) + q]) atomicOr(fail + ui, 1u);
+  if (!g.live) return;
+  if (!g.last) {
+    if (v != next) atomicOr(fail + g.ui, 1u);
   } else if (q == 0) {
-    if (xfinal(all, total, tail, tail_len) != un->digest) atomicOr(fail + ui, 1u);
+    if (xfinal(all, g.total, g.tail) != g.digest) atomicOr(fail + g.ui, 1u);
   }
 }
 
-// Device-gated verify: one quad per (unit, segment) of the launch's units, all of the arena's part shape. kCopy (the
-// staged units' fused scatter): unit u's bytes are read from src + u x unit_bytes, where its parts lie back to back,
-// and written to their arena slot as they are hashed; the last segment's lane 0 also moves the unit's tail.
+// Device-gated verify: one quad per segment of a unit, the launch's units (all of the arena's part shape) along the
+// grid's y, so that a wave has one unit: its key and slot are scalar, and no segment index is divided. kCopy (the staged
+// units' fused scatter): unit u's bytes are read from src + u x unit_bytes, where its parts lie back to back, and
+// written to their arena slot as they are hashed; the last segment's lane 0 also moves the unit's tail.
 struct DgSeg {
-  uint64_t v = 0, local = 0, key = 0;
-  uint32_t u = 0, stripes = 0, tail_len = 0;
+  const uint64_t* state = nullptr;
+  uint64_t digest = 0;
+  uint32_t stripes = 0;
   bool live = false, last = false;
   const unsigned char* from = nullptr;  // the segment's first byte (where it is read)
   unsigned char* to = nullptr;          // (kCopy) where it is written
-  const unsigned char* tail = nullptr;
+  const unsigned char* tail = nullptr;  // (last) the bytes after the last stripe, and where they are written
+  unsigned char* tail_to = nullptr;
+  uint32_t tail_len = 0;
 };
 
-// The launch's tables (keys, slots, the parts' arrays) are kernel arguments. Indexed by a per-lane value they become
-// per-lane loads from the argument segment; so the wave reads its first lane's unit with scalar loads (per-lane
-// loads only run in a wave that straddles two units) and the part's fields are carried along the walk over the parts
-// with constant indices, which keeps every other read of the arguments a scalar load.
-
+// (The part's fields are carried along the walk over the parts with constant indices, which keeps every read of the
+// launch's arguments a scalar load.)
 template <bool kCopy>
-__device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsigned char* src, uint64_t s, uint32_t q) {
+__device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsigned char* src, uint64_t local) {
   DgSeg g;
-  g.live = s < uint64_t(a.n) * a.unit_segs;
-  const uint32_t u_lane = g.live ? uint32_t(s / a.unit_segs) : a.n - 1;  // (a dead lane sides with the last unit)
-  const uint32_t u0 = __builtin_amdgcn_readfirstlane(u_lane);
-  uint32_t key = a.keys[u0];  // scalar loads, here (the empty asm takes them as scalars before any branch)
-  int32_t slot = a.slots[u0];
-  asm volatile("" ::"s"(key), "s"(slot));
-  if (!__all(u_lane == u0)) {  // only in a wave that straddles two units
-    key = a.keys[u_lane];
-    slot = a.slots[u_lane];
-  }
+  const uint32_t u = blockIdx.y;
+  const uint64_t key = a.keys[u];
+  const int32_t slot = a.slots[u];
+  g.live = local < a.unit_segs;
   if (!g.live) return g;
-  g.u = u_lane;
-  g.local = s - uint64_t(g.u) * a.unit_segs;
-  uint64_t k = g.local;
+  g.state = a.ckpt + (key * a.unit_segs + local) * 4;
+  g.digest = a.digests[key];
+  uint64_t k = local;
   uint32_t p = 0;
-  uint64_t src_off = uint64_t(g.u) * a.unit_bytes;  // (kCopy) the part's first byte in src
+  uint64_t src_off = uint64_t(u) * a.unit_bytes;  // (kCopy) the part's first byte in src
   uint64_t pbytes = a.part_bytes[0], psegs = a.part_segs[0];
   const unsigned char* parena = a.arena[0];
 #pragma unroll
@@ -666,33 +864,34 @@ __device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsig
   unsigned char* base = const_cast<unsigned char*>(parena) + uint64_t(slot) * pbytes;
   const unsigned char* from = kCopy ? src + src_off : base;
   g.last = last_part && k + 1 == psegs;
-  if (g.last) {
-    g.tail = from + span;
-    g.tail_len = uint32_t(pbytes - span);
-    if (kCopy && q == 0)
-      for (uint32_t i = 0; i < g.tail_len; ++i) base[span + i] = g.tail[i];
-  }
-  g.key = key;
-  g.v = a.ckpt[(g.key * a.unit_segs + g.local) * 4 + q];
+  g.tail = from + span;
+  g.tail_to = base + span;
+  g.tail_len = uint32_t(pbytes - span);
+  g.stripes = end > off ? uint32_t((end - off) / 32) : 0;
   g.from = from + off;
   g.to = base + off;
-  g.stripes = end > off ? uint32_t((end - off) / 32) : 0;
   return g;
 }
 
 // The segment's check (the next checkpoint, or for the unit's last segment the digest) and the gate.
-__device__ __forceinline__ void dg_finish(const DgVerifyLaunch& a, const DgSeg& g, uint64_t v, uint32_t q) {
+template <bool kCopy>
+__device__ __forceinline__ void dg_finish(const DgVerifyLaunch& a, const DgSeg& g, const Tail& tail, uint64_t v, uint64_t next,
+                                          uint32_t q) {
   uint64_t all[4];
   const uint32_t base4 = threadIdx.x & ~3u;
 #pragma unroll
   for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int(base4 + k), 64);
   bool bad = false;
   if (g.live) {
-    if (!g.last) bad = v != a.ckpt[(g.key * a.unit_segs + g.local + 1) * 4 + q];
-    else if (q == 0) bad = xfinal(all, a.unit_bytes, g.tail, g.tail_len) != a.digests[g.key];
+    if (!g.last) {
+      bad = v != next;
+    } else if (q == 0) {
+      bad = xfinal(all, a.unit_bytes, tail) != g.digest;
+      if (kCopy) store_tail(g.tail_to, tail);
+    }
   }
   if (bad) {
-    atomicOr(a.fail + g.u, 1u);
+    atomicOr(a.fail + blockIdx.y, 1u);
     if (a.abort) {  // the gate: the token fails before the layer's ready word is written
       if (atomicCAS(a.err_code, 0u, a.err) == 0u) atomicExch(a.err_aux, a.aux);
       atomicExch(a.abort, 1u);
@@ -717,37 +916,50 @@ __global__ __launch_bounds__(64) void dg_publish_kernel(const DgVerifyLaunch a) 
 }
 
 template <bool kCopy>
-__device__ __forceinline__ void dg_verify_body(const DgVerifyLaunch& a, const unsigned char* src) {
+__device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, const unsigned char* src) {
   const uint64_t gid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const uint32_t q = uint32_t(gid & 3u);
-  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2, q);
-  uint64_t v = 0;
-  if (g.live) v = chain_t<kCopy>(g.v, g.from, g.to, g.stripes, q);
-  dg_finish(a, g, v, q);
+  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
+  uint64_t v = 0, next = 0;
+  if (g.live) {
+    next = g.last ? 0 : g.state[4 + q];
+    v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
+  }
+  Tail tail;
+  if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
+  dg_finish<kCopy>(a, g, tail, v, next, q);
 }
-
-__global__ TSA_VERIFY_BOUNDS void dg_verify_kernel(const DgVerifyLaunch a) { dg_verify_body<false>(a, nullptr); }
+__global__ TSA_VERIFY_BOUNDS void dg_verify_kernel(const DgVerifyLaunch a) { dg_chain_body<false>(a, nullptr); }
 __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_verify_body<true>(a, src);
+  dg_chain_body<true>(a, src);
 }
 
-template <bool kCopy>
-__device__ __forceinline__ void dg_verify_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kLdsWaveBytes];
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  unsigned char* mine = lds + wave * kLdsWaveBytes;
-  const uint32_t mine_off = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(mine)));
-  const uint64_t gid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+template <uint32_t kD, bool kNt, uint32_t kThreads, bool kCopy>
+__device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kThreads / 64 * lds_bytes<kD>()];
+  const uint64_t gid = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
+  if ((gid & ~63ull) >> 2 >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = uint32_t(gid & 3u);
-  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2, q);
-  // a dead quad (past the launch's segments) streams unit 0's first bytes and hashes (and writes) none of them
-  const unsigned char* from = g.live ? g.from : kCopy ? src : a.arena[0] + uint64_t(a.slots[0]) * a.part_bytes[0];
-  const uint64_t v = lds_chain_t<kCopy>(g.v, from, g.to, g.live ? g.stripes : 0u, mine, mine_off);
-  dg_finish(a, g, v, q);
+  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
+  Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
+  if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
+  uint64_t v = 0, next = 0;
+  if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
+    v = lds_check<kD, kNt, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+                                  g.state, g.last, wave_lds(lds, lds_bytes<kD>()), &next);
+  } else if (g.live) {
+    next = g.last ? 0 : g.state[4 + q];
+    v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
+  }
+  dg_finish<kCopy>(a, g, tail, v, next, q);
 }
-__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) { dg_verify_lds_body<false>(a, nullptr); }
-__global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_verify_lds_body<true>(a, src);
+template <uint32_t kD, bool kNt, uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
+  dg_lds_body<kD, kNt, kThreads, false>(a, nullptr);
+}
+template <bool kNt, uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
+  dg_lds_body<2, kNt, kThreads, true>(a, src);
 }
 
 }  // namespace dev
@@ -774,17 +986,24 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
   return int(hipGetLastError());
 }
 
-// The LDS-streamed kernel needs 2 KiB segments and every part of every unit of the launch 16-byte aligned and at
-// least 16 bytes long (a lane with nothing to load reads its segment's first 16 bytes).
-static bool dg_lds_shape(const DgVerifyLaunch& a) {
-  if (a.seg_bytes != dev::kLdsSegBytes) return false;
-  for (uint32_t p = 0; p < a.n_parts; ++p) {
-    if (reinterpret_cast<uintptr_t>(a.arena[p]) % 16 != 0 || a.part_bytes[p] < 16) return false;
-    if (a.part_bytes[p] % 16 == 0) continue;
-    for (uint32_t u = 0; u < a.n; ++u)
-      if (uint64_t(a.slots[u]) * a.part_bytes[p] % 16 != 0) return false;
-  }
-  return true;
+// How a launch of `waves` waves of 16 segments that touches `bytes` (the copy: twice its units') runs.
+//  * Segments of no whole number of chunk pairs, or longer than 4 KiB: the chain loop (one 24.8 MB unit, 8 KiB segments:
+//    13.1 us; a wave's pieces then lie far apart, and with 4 KiB segments beyond the caches streaming already loses:
+//    122 MB 26.5 us against 23.3).
+//  * Up to 512 waves, two per CU: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us
+//    against 5.2; 8 MiB 5.3 / 5.7). From about 750 waves the workgroups' 33 KiB of LDS no longer lie evenly over the
+//    CUs (24.8 MB: 7.5 against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
+//  * Up to 80 MB touched: cached loads, in workgroups of one wave. The bytes have just landed, and the engine reads
+//    them next: a non-temporal read of what the caches hold is the slower one (staged 24.8 MB unit, the buffers
+//    changing from pass to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6). Above, whole lines with the
+//    non-temporal hint read faster (336 MiB unit: 55 us against 60; 98.8 MB of odd units 19.0 / 20.4).
+enum class Stream { kChain, kAll4, kAll8, kCached, kNt };
+static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
+  const bool far = bytes > 80000000;
+  if (seg_bytes % 512 != 0 || seg_bytes > 4096 || (seg_bytes > 2048 && far)) return Stream::kChain;
+  if (!copy && waves <= 512 && seg_bytes == 2048) return Stream::kAll8;
+  if (!copy && waves <= 512 && seg_bytes == 1024) return Stream::kAll4;
+  return far ? Stream::kNt : Stream::kCached;
 }
 
 static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
@@ -793,59 +1012,64 @@ static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
   return int(hipGetLastError());
 }
 
+// start and stop (both or neither) take the dispatch's own begin and end timestamps.
+template <class K, class... A>
+static int launch_timed(K* k, dim3 grid, uint32_t threads, hipStream_t stream, hipEvent_t start, hipEvent_t stop,
+                        const A&... args) {
+  if (start && stop)
+    hipExtLaunchKernelGGL(k, grid, dim3(threads), 0, stream, start, stop, 0, args...);
+  else
+    hipLaunchKernelGGL(k, grid, dim3(threads), 0, stream, args...);
+  return int(hipGetLastError());
+}
+
 int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4) return int(hipErrorInvalidValue);
-  const uint32_t threads = 256;
-  const uint64_t blocks = (uint64_t(a.n) * a.unit_segs * 4 + threads - 1) / threads;
-  if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
-  auto* k = dg_lds_shape(a) ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
-  if (start && stop)  // the events take the dispatch's own begin and end timestamps
-    hipExtLaunchKernelGGL(k, dim3(uint32_t(blocks)), dim3(threads), 0, stream, start, stop, 0, a);
-  else
-    hipLaunchKernelGGL(k, dim3(uint32_t(blocks)), dim3(threads), 0, stream, a);
-  const int e = int(hipGetLastError());
+  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), a.n * a.unit_bytes, false);
+  const uint32_t threads = rule == Stream::kChain || rule == Stream::kNt ? 256 : 64;
+  const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
+  if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
+  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false, 64>
+            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false, 64>
+            : rule == Stream::kCached ? dev::dg_verify_lds_kernel<2, false, 64>
+            : rule == Stream::kNt     ? dev::dg_verify_lds_kernel<2, true, 256>
+                                      : dev::dg_verify_kernel;
+  const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
-}
-
-// The fused kernel's LDS form also needs the staged bytes 16-byte aligned: src and every part of every staged unit.
-static bool dg_scatter_lds_shape(const DgVerifyLaunch& a, const void* src) {
-  if (!dg_lds_shape(a) || reinterpret_cast<uintptr_t>(src) % 16 != 0) return false;
-  for (uint32_t p = 0; p < a.n_parts; ++p)
-    if (a.part_bytes[p] % 16 != 0) return false;
-  return true;
 }
 
 int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream_t stream, hipEvent_t start,
                              hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
-  const uint32_t threads = 256;
-  const uint64_t blocks = (uint64_t(a.n) * a.unit_segs * 4 + threads - 1) / threads;
-  if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
-  const unsigned char* s = static_cast<const unsigned char*>(src);
-  auto* k = dg_scatter_lds_shape(a, src) ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
-  if (start && stop)
-    hipExtLaunchKernelGGL(k, dim3(uint32_t(blocks)), dim3(threads), 0, stream, start, stop, 0, a, s);
-  else
-    hipLaunchKernelGGL(k, dim3(uint32_t(blocks)), dim3(threads), 0, stream, a, s);
-  const int e = int(hipGetLastError());
+  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), 2 * a.n * a.unit_bytes, true);
+  const uint32_t threads = rule == Stream::kCached ? 64 : 256;
+  const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
+  if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
+  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<false, 64>
+            : rule == Stream::kNt   ? dev::dg_scatter_verify_lds_kernel<true, 256>
+                                    : dev::dg_scatter_verify_kernel;
+  const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
+                             static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
 }
 
 int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_segments, uint64_t seg_bytes,
                   uint32_t* fail_dev, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (n_units == 0 || n_segments == 0) return 0;
-  const uint32_t threads = 256;
+  const Stream rule = stream_rule(seg_bytes, (n_segments + 15) / 16, n_segments * seg_bytes, false);
+  const uint32_t threads = rule == Stream::kChain || rule == Stream::kNt ? 256 : 64;
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
-  if (start && stop)  // the events take the dispatch's own begin and end timestamps
-    hipExtLaunchKernelGGL(dev::verify_kernel, dim3(uint32_t(blocks)), dim3(threads), 0, stream, start, stop, 0,
-                          units_dev, n_units, n_segments, seg_bytes, fail_dev);
-  else
-    hipLaunchKernelGGL(dev::verify_kernel, dim3(uint32_t(blocks)), dim3(threads), 0, stream, units_dev, n_units,
-                       n_segments, seg_bytes, fail_dev);
-  return int(hipGetLastError());
+  const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
+  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, 64>
+            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, 64>
+            : rule == Stream::kCached ? dev::verify_kernel<2, false, 64>
+            : rule == Stream::kNt     ? dev::verify_kernel<2, true, 256>
+                                      : dev::verify_kernel<0, false, 256>;
+  return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
+                      shift, fail_dev);
 }
 
 }  // namespace tsa
