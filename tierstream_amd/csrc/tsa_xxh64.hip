@@ -122,8 +122,8 @@ __device__ __forceinline__ uint64_t xfinal(const uint64_t v[4], uint64_t total, 
 // Measured on one 336 MiB unit (8 KiB segments): this loop reads at 5.8 TB/s, 95 % of what a fully coalesced 16-byte
 // streaming read of the same bytes reaches in one launch (6.1 TB/s); the rounds alone (no loads) run at 17 TB/s. So
 // the kernel is bound by the read, not the multiplies, and neither a software-pipelined nor an LDS-staged variant
-// (coalesced 16-byte loads into LDS, chains run from LDS) beat it. Sixteen stripes a block: with 32 or 64 in registers
-// (one or two memory latencies a segment) 25 MB of 8-byte aligned units took 8.2 and 9.5 us against 7.6.
+// (coalesced 16-byte loads into LDS, chains run from LDS) beat it. Sixteen stripes a block: with 8, 25 MB of
+// 8-byte aligned units took 8.3 us against 7.6; with 32, 34 MB of ragged ones 12.0 against 10.7.
 constexpr int kBlock = 16;
 
 // kCopy: each word read is also stored at the same offset from d (the staged unit's bytes into their arena slot while
