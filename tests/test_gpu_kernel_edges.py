@@ -166,3 +166,32 @@ def test_batch_checks_by_shape(gpu, n, parts, seg, align):
         gpu.check(gpu.lib().tsa_xxh64_verify(C.c_void_p(table.ptr), n, first, seg, C.c_void_p(fail.ptr), None))
         gpu.check(gpu.lib().tsa_stream_sync(None))
         assert list(fail.download(4 * n).view(np.uint32)) == want
+
+
+# 16 KiB blocks part by part; more jobs than a wave's 64 probes; near (cached) and, above 80 MB moved, far launches.
+@pytest.mark.parametrize("n,parts", [(1, [16]), (1, [16384]), (2, [16400, 32, 0, 16368]), (65, [16384 * 3, 48]),
+                                     (200, [1024, 16]), (3, [13 << 20, (1 << 20) + 16])])
+def test_scatter_jobs(gpu, n, parts):
+    rng = np.random.default_rng(n + sum(parts))
+    ub = sum(parts)
+    host = rng.integers(0, 256, (n, ub), dtype=np.uint8)
+    src, bufs = gpu.DeviceBuffer(host.nbytes), [gpu.DeviceBuffer((n + 1) * max(p, 16)) for p in parts]
+    src.upload(host.reshape(-1))
+    for buf, p in zip(bufs, parts):
+        buf.upload(np.zeros((n + 1) * max(p, 16), dtype=np.uint8))
+    per = int(gpu.lib().tsa_scatter_blocks((C.c_uint64 * len(parts))(*parts), len(parts)))
+    slots, jobs = rng.permutation(n + 1)[:n], []
+    for i in range(n):
+        j = gpu.TsaScatterJob()
+        j.src, j.n_parts, j.block_first = src.ptr + i * ub, len(parts), i * per
+        for p, (buf, pb) in enumerate(zip(bufs, parts)):
+            j.dst[p], j.bytes[p] = buf.ptr + int(slots[i]) * pb, pb
+        jobs.append(j)
+    table = gpu.upload_struct_array(jobs)
+    gpu.check(gpu.lib().tsa_scatter(C.c_void_p(table.ptr), n, n * per, None))
+    gpu.check(gpu.lib().tsa_stream_sync(None))
+    cuts = np.cumsum([0] + parts)
+    for p, buf in enumerate(bufs):
+        want = np.zeros((n + 1, parts[p]), dtype=np.uint8)
+        want[slots] = host[:, cuts[p]:cuts[p + 1]]
+        assert np.array_equal(buf.download()[:want.size].reshape(want.shape), want)

@@ -16,6 +16,7 @@
 #include <stdint.h>
 
 #include "tsa_device.hpp"
+#include "wave_search.hpp"
 
 namespace tsa {
 namespace dev {
@@ -699,19 +700,6 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
 // not in registers.
 #define TSA_VERIFY_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
 
-// The last unit of [0, n_units) whose seg_first is at most s (ascending): 64 probes at a time.
-__device__ __forceinline__ uint32_t unit_of(const TsaVerifyUnit* units, uint32_t n_units, uint64_t s) {
-  uint32_t lo = 0, hi = n_units;
-  while (hi - lo > 1) {
-    const uint32_t step = (hi - lo + 63) / 64, at = lo + (threadIdx.x & 63u) * step;
-    const bool under = at < hi && at >= lo && units[at].seg_first <= s;
-    const uint32_t k = uint32_t(__popcll(__ballot(under)));
-    lo += (k ? k - 1 : 0) * step;
-    hi = hi - lo < step ? hi : lo + step;
-  }
-  return lo;
-}
-
 // A segment of a unit given by its extents: where it lies and what it must lead to.
 struct HostSeg {
   const unsigned char* from = nullptr;
@@ -776,7 +764,7 @@ __global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* _
   const uint32_t q = threadIdx.x & 3u;
   const uint64_t s = s0 + ((threadIdx.x & 63u) >> 2);
   const uint64_t end = n_segments - s0 < 16 ? n_segments : s0 + 16;
-  uint32_t ui = unit_of(units, n_units, s0);
+  uint32_t ui = last_at_most(n_units, s0, [&](uint32_t i) { return units[i].seg_first; });
   HostSeg g;
   const uint64_t after = ui + 1 < n_units ? units[ui + 1].seg_first : ~0ull;
   const TsaVerifyUnit un = units[ui];  // (whole and at once: with scalar loads, one memory latency)
