@@ -20,7 +20,14 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr uint64_t kChunk = 256 * 1024;  // bytes per workgroup
+
+// Bytes per workgroup of a layer's read: 256 KiB, less where its units would then give fewer than four workgroups a CU
+// (two units of 3 MiB were 24 workgroups of 16 serial reads).
+uint64_t chunk_of(uint64_t unit_bytes, uint32_t units) {
+  uint64_t c = 256 * 1024;
+  while (c > 16 * 1024 && unit_bytes / c * units < 1024) c /= 2;
+  return c;
+}
 
 // Words [first_word, first_word + n_words) of a unit, read from p (16-byte aligned; units below 16 GiB, so word indexes
 // fit 32 bits). The read is shaped like a batch-1 expert GEMV's: 16-byte loads, four per lane in flight, every byte
@@ -71,18 +78,19 @@ __device__ __forceinline__ void block_add(uint64_t s, unsigned long long* out) {
 
 // Host contract: blockIdx.y = routed unit i (its table entry table_dev[ids[i]]); blockIdx.x = a chunk of its bytes.
 __global__ __launch_bounds__(kThreads) void checksum_table(const uint64_t* table_dev, const int32_t* ids, uint64_t bytes,
-                                                           unsigned long long* out) {
+                                                           uint64_t chunk, unsigned long long* out) {
   const int32_t u = ids[blockIdx.y];
   const uint64_t a = table_dev[u];
-  const uint64_t off = uint64_t(blockIdx.x) * kChunk;
+  const uint64_t off = uint64_t(blockIdx.x) * chunk;
   if (a == 0 || off >= bytes) return;
-  const uint64_t n = (bytes - off < kChunk ? bytes - off : kChunk) / 4;
+  const uint64_t n = (bytes - off < chunk ? bytes - off : chunk) / 4;
   block_add(sum_words(reinterpret_cast<const uint32_t*>(a + off), off / 4, n), out + blockIdx.y);
 }
 
 // Device-gated: the slot from ss_dg_slot, then each part at base + slot * stride.
 __global__ __launch_bounds__(kThreads) void checksum_dg(ss_dg_device_view v, uint32_t g, const int32_t* ids,
-                                                        unsigned long long* out, unsigned long long* start) {
+                                                        uint64_t chunk, unsigned long long* out,
+                                                        unsigned long long* start) {
   __shared__ int32_t slot_s;
   if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0) start[g] = wall_clock64();  // the layer's compute began
   if (threadIdx.x == 0) slot_s = ss_dg_slot(&v, g, ids[blockIdx.y]);
@@ -90,10 +98,10 @@ __global__ __launch_bounds__(kThreads) void checksum_dg(ss_dg_device_view v, uin
   const int32_t slot = slot_s;
   uint64_t b = blockIdx.x, word0 = 0;
   for (uint32_t p = 0; p < v.n_parts; ++p) {  // chunk b of the unit: each part has its own whole chunks
-    const uint64_t pb = v.parts[p].bytes, nb = (pb + kChunk - 1) / kChunk;
+    const uint64_t pb = v.parts[p].bytes, nb = (pb + chunk - 1) / chunk;
     if (b < nb) {
-      const uint64_t off = b * kChunk;
-      const uint64_t n = (pb - off < kChunk ? pb - off : kChunk) / 4;
+      const uint64_t off = b * chunk;
+      const uint64_t n = (pb - off < chunk ? pb - off : chunk) / 4;
       const uint32_t* base = reinterpret_cast<const uint32_t*>(static_cast<const char*>(v.parts[p].base) +
                                                                uint64_t(slot) * v.parts[p].stride + off);
       block_add(sum_words(base, word0 + off / 4, n), out + blockIdx.y);
@@ -133,7 +141,7 @@ ss_status ck(hipError_t e) { return e == hipSuccess ? SS_OK : SS_E_BACKEND; }
   } while (0)
 #define TSE_HIP(x) TSE_CK(ck(x))
 
-uint32_t chunks_of(uint64_t bytes) { return uint32_t((bytes + kChunk - 1) / kChunk); }
+uint32_t chunks_of(uint64_t bytes, uint64_t chunk) { return uint32_t((bytes + chunk - 1) / chunk); }
 
 double ms_since(std::chrono::steady_clock::time_point t) {
   return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
@@ -215,8 +223,9 @@ __attribute__((visibility("default"))) ss_status tse_host_run_ex(ss_ctx* c, cons
       if (n_read > 0) {
         st = ck(hipMemcpyAsync(ids_dev + size_t(l) * max_ids, rid, 4ull * n_read, hipMemcpyHostToDevice, s));
         if (st == SS_OK) {
-          hipLaunchKernelGGL(checksum_table, dim3(chunks_of(ss_desc_unit_bytes(d, l)), n_read), dim3(kThreads), 0, s,
-                             v.table_dev, ids_dev + size_t(l) * max_ids, ss_desc_unit_bytes(d, l),
+          const uint64_t bytes = ss_desc_unit_bytes(d, l), chunk = chunk_of(bytes, uint32_t(n_read));
+          hipLaunchKernelGGL(checksum_table, dim3(chunks_of(bytes, chunk), n_read), dim3(kThreads), 0, s,
+                             v.table_dev, ids_dev + size_t(l) * max_ids, bytes, chunk,
                              out_dev + size_t(l) * max_ids);
           st = ck(hipGetLastError());
         }
@@ -268,6 +277,7 @@ __attribute__((visibility("default"))) ss_status tse_host_run(ss_ctx* c, const s
 struct TseDg {
   ss_ctx* c = nullptr;
   uint32_t G = 0, n_ids = 0, max_chunks = 0;
+  uint64_t chunk = 0;
   uint32_t n_pred = 0;  // ids predicted at each layer for the next one (0: no predictions)
   uint32_t rows = 1;  // the verify rows each token closes (above one: ss_dg_end_rows instead of ss_end)
   bool checksum = true, dg = true;
@@ -311,7 +321,7 @@ static ss_status tse_enqueue_token(TseDg* e) {
     if (e->dg) TSE_CK(ss_dg_enqueue_wait(e->c, int(g), e->s));
     if (e->checksum) {
       hipLaunchKernelGGL(checksum_dg, dim3(e->max_chunks, e->n_ids), dim3(kThreads), 0, e->s, e->view, g,
-                         e->ids_dev + 64 * g, e->out_dev + 64 * g, e->start_dev);
+                         e->ids_dev + 64 * g, e->chunk, e->out_dev + 64 * g, e->start_dev);
       TSE_HIP(hipGetLastError());
     }
   }
@@ -358,9 +368,10 @@ __attribute__((visibility("default"))) ss_status tse_dg_create_ex(ss_ctx* c, uin
     return st;
   }
   e->G = e->view.n_gated;
-  uint32_t chunks = 0;
-  for (uint32_t p = 0; p < e->view.n_parts; ++p) chunks += chunks_of(e->view.parts[p].bytes);
-  e->max_chunks = chunks;
+  uint64_t bytes = 0;
+  for (uint32_t p = 0; p < e->view.n_parts; ++p) bytes += e->view.parts[p].bytes;
+  e->chunk = chunk_of(bytes, n_ids);
+  for (uint32_t p = 0; p < e->view.n_parts; ++p) e->max_chunks += chunks_of(e->view.parts[p].bytes, e->chunk);
   if (hipStreamCreateWithFlags(&e->s, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&e->ids_dev, 4ull * 64 * e->G) != hipSuccess || hipMalloc(&e->pred_dev, 4ull * 64 * e->G) != hipSuccess ||
       hipMalloc(&e->out_dev, 8ull * 64 * e->G) != hipSuccess ||
