@@ -60,12 +60,13 @@ def test_synth_edges(gpu, kind, words, offset):
 
 
 # The checks by segment size and by size: all chunks of a wave in flight (1 and 2 KiB segments, up to 512 waves), two
-# chunk buffers (whole pairs of 256-byte chunks), non-temporal reads (above 80 MB), the chain loop (other segments;
-# waves with a segment that is 8-byte aligned); parts that end inside a segment, inside a stripe, or are none.
+# chunk buffers (whole pairs of 256-byte chunks), four with non-temporal reads (above 80 MB; non-temporal stores too
+# above 256 MiB moved), the chain loop (other segments; waves with a segment that is 8-byte aligned); parts that end
+# inside a segment, inside a stripe, or are none.
 SHAPES = [
     (1, [2048], 2048), (1, [32], 2048), (2, [8], 2048), (1, [2080, 40], 2048), (5, [65568, 4096, 1000], 2048),
     (64, [30 * 2048 + 32, 96], 2048), (3, [2048 * 17, 2048 * 15 + 64, 32, 2048], 2048), (3, [(8 << 20) + 32, 1 << 20], 2048),
-    (3, [28 << 20, (3 << 20) + 48], 2048), (2, [65536, 2048 + 1008], 512), (3, [65536 + 96, 1024 * 16], 1024),
+    (3, [28 << 20, (3 << 20) + 48], 2048), (3, [45 << 20, 4096 + 24], 2048), (2, [65536, 2048 + 1008], 512), (3, [65536 + 96, 1024 * 16], 1024),
     (2, [9 << 20, 1024 * 3 + 8], 1024), (3, [1536 * 40 + 32, 1536 * 16 - 8], 1536), (2, [1 << 20, 4096 * 3 + 56], 4096),
     (3, [28 << 20, 4096 + 16], 4096), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
 ]

@@ -453,8 +453,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
 constexpr uint32_t kStateBytes = 1024;  // per wave, at the end of its LDS: 64 bytes per quad
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
-typedef __attribute__((address_space(1))) u32x4_a8 gu32x4_t;
+typedef __attribute__((address_space(1))) u32x4 gu32x4_t;
 
 // M0 (the LDS destination) is restored for the compiler; s_nop: an M0 write before a load to LDS.
 #define TSA_LDS_LOAD16(HINT)                         \
@@ -513,16 +512,6 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// A wave's part of its workgroup's LDS: its address and its 32-bit LDS address.
-struct WaveLds {
-  unsigned char* p;
-  uint32_t off;
-};
-__device__ __forceinline__ WaveLds wave_lds(unsigned char* lds, uint32_t bytes) {
-  unsigned char* p = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * bytes;
-  return {p, uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(p)))};
-}
-
 template <uint32_t kD, bool kNt, uint32_t kC = 0>
 __device__ __forceinline__ void issue_all(const unsigned char* const g[4], uint32_t lds_off) {
   if constexpr (kC < kD) {
@@ -543,21 +532,21 @@ __device__ __forceinline__ void drain(F&& hash) {
 // One wave's 16 segments (quad j's lanes 4 j + q hold segment j): where it is read and (kCopy) written, its stripes (0
 // hashes nothing and reads 16 bytes), its checkpoint (32 bytes, 64 when it is not the unit's last). Out: the
 // accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
-// go along with the first live segment and their results mean nothing. The wave's LDS has lds_bytes<kD>().
+// go along with the first live segment and their results mean nothing. The workgroup is one wave, with lds_bytes<kD>().
 //
-// kD = 2: two chunk buffers, chunk c+2 loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0). kD > 2:
-// segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy, whose stores
-// the waits would wait for).
+// kRing: kD chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt
+// 0). Otherwise segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy,
+// whose stores the waits would wait for). kNt: reads go past the caches, kNtStore: the
+// copy's stores do.
 template <uint32_t kD>
 constexpr uint32_t lds_bytes() {
   return kD * 4096 + kStateBytes;
 }
-template <uint32_t kD, bool kNt, bool kCopy>
+template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
                                               uint32_t stripes, const uint64_t* state, bool last,
-                                              const WaveLds& w, uint64_t* next) {
-  const unsigned char* lds = w.p;
-  const uint32_t lds_off = w.off;
+                                              unsigned char* lds, uint64_t* next) {
+  const uint32_t lds_off = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(lds)));
   const uint32_t lane = threadIdx.x & 63u, q = lane & 3u, j = lane >> 2;
   const uint32_t i = lane >> 4, m = lane & 15u;
   const int first = __ffsll(static_cast<long long>(__ballot(live))) - 1;
@@ -568,13 +557,13 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
   from = reinterpret_cast<const unsigned char*>(from_first(reinterpret_cast<uintptr_t>(from), reinterpret_cast<uintptr_t>(from)));
   state = reinterpret_cast<const uint64_t*>(from_first(reinterpret_cast<uintptr_t>(state), reinterpret_cast<uintptr_t>(state)));
   last = last || !live;
-  static_assert(kD == 2 || !kCopy, "");
+  static_assert(kRing || !kCopy, "");
   uint32_t chunks = kD;
-  if (kD == 2) {  // as many pairs as the wave's longest segment has
+  if (kRing) {  // as many rounds of the buffers as the wave's longest segment has
     uint32_t most = stripes;
 #pragma unroll
     for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
-    chunks = max(2u, __builtin_amdgcn_readfirstlane((most + 15) / 16 * 2));
+    chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
   }
   const bool whole = __all(!live || stripes == 8 * chunks);
   lds_load16<kNt>(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
@@ -604,19 +593,25 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     for (uint32_t k = 0; k < 4; ++k) g[k] = src[k] + min(256 * c, lim[k]);
     lds_load_chunk<0, kNt>(g, lds_off + buf * 4096);
   };
+  auto put = [](unsigned char* p, u32x4 x) {  // (a global store: a generic one would also count on the LDS counter)
+    gu32x4_t* at = reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(p));
+    if (kNtStore)
+      __builtin_nontemporal_store(x, at);
+    else
+      *at = x;
+  };
   const bool full = kCopy && __all(live && stripes == 8 * chunks);
   auto store = [&](uint32_t c, uint32_t buf) {  // the lane's own four pieces, as they landed in LDS
     u32x4 x[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const u32x4*>(lds + buf * 4096 + k * 1024 + lane * 16);
-    // (global stores: a generic one would also count on the LDS counter)
     if (full) {
 #pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(dst[k] + c * 256)) = x[k];
+      for (uint32_t k = 0; k < 4; ++k) put(dst[k] + c * 256, x[k]);
     } else {
 #pragma unroll
       for (uint32_t k = 0; k < 4; ++k)
-        if (g0[k] + 8 * c < n[k]) *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(dst[k] + c * 256)) = x[k];
+        if (g0[k] + 8 * c < n[k]) put(dst[k] + c * 256, x[k]);
     }
   };
   const uint32_t rot = j & 7u;
@@ -647,7 +642,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     b = st[q] * P1inv;
     *next = st[4 + q];
   };
-  if constexpr (kD == 2) {
+  if constexpr (kRing) {
     auto issue = [&](uint32_t c, uint32_t buf) {
       if (whole) {
         lds_load_chunk<0, kNt>(src, lds_off + buf * 4096);
@@ -657,28 +652,25 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
         issue_part(c, buf);
       }
     };
-    issue(0, 0);
-    issue(1, 1);
-    wait_loads<8>();
+#pragma unroll
+    for (uint32_t c = 0; c < kD; ++c) issue(c, c);
+    wait_loads<4 * kD>();
     states();
-    for (uint32_t c = 0; c + 2 < chunks; c += 2) {
-      wait_loads<4>();
-      if (kCopy) store(c, 0);
-      hash(c, 0);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue(c + 2, 0);
-      wait_loads<4>();
-      if (kCopy) store(c + 1, 1);
-      hash(c + 1, 1);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue(c + 3, 1);
+    for (uint32_t c = 0; c + kD < chunks; c += kD) {
+#pragma unroll
+      for (uint32_t i = 0; i < kD; ++i) {
+        wait_loads<4 * (kD - 1)>();
+        if (kCopy) store(c + i, i);
+        hash(c + i, i);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(c + i + kD, i);
+      }
     }
-    wait_loads<4>();
-    if (kCopy) store(chunks - 2, 0);
-    hash(chunks - 2, 0);
-    wait_loads<0>();
-    if (kCopy) store(chunks - 1, 1);
-    hash(chunks - 1, 1);
+    const uint32_t c = chunks - kD;
+    drain<kD>([&](uint32_t i) {
+      if (kCopy) store(c + i, i);
+      hash(c + i, i);
+    });
   } else {
     if (whole) {
       issue_all<kD, kNt>(src, lds_off);
@@ -755,7 +747,7 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
 }
 // One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
 // lds_check; 0 runs the chain loop from memory.
-template <uint32_t kD, bool kNt, uint32_t kThreads>
+template <uint32_t kD, bool kRing, bool kNt, uint32_t kThreads>
 __global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
                                                           uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
                                                           uint32_t* __restrict__ fail) {
@@ -780,10 +772,10 @@ __global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* _
   bool streamed = false;
   if constexpr (kD != 0) {
     streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kThreads / 64 * lds_bytes<kD>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes<kD>()];  // (one wave)
     if (streamed)
-      v = lds_check<kD, kNt, false>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr,
-                                    g.stripes, g.state, g.last, wave_lds(lds, lds_bytes<kD>()), &next);
+      v = lds_check<kD, kRing, kNt, false, false>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr,
+                                    g.stripes, g.state, g.last, lds, &next);
   }
   if (!streamed && g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -922,32 +914,31 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
   dg_chain_body<true>(a, src);
 }
 
-template <uint32_t kD, bool kNt, uint32_t kThreads, bool kCopy>
+template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kThreads / 64 * lds_bytes<kD>()];
-  const uint64_t gid = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if ((gid & ~63ull) >> 2 >= a.unit_segs) return;  // (the whole wave)
+  __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes<kD>()];
+  const uint64_t gid = uint64_t(blockIdx.x) * 64 + threadIdx.x;
   const uint32_t q = uint32_t(gid & 3u);
   const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
   Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
-    v = lds_check<kD, kNt, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
-                                  g.state, g.last, wave_lds(lds, lds_bytes<kD>()), &next);
+    v = lds_check<kD, kRing, kNt, kCopy, kNtStore>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+                                  g.state, g.last, lds, &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
     v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
   }
   dg_finish<kCopy>(a, g, tail, v, next, q);
 }
-template <uint32_t kD, bool kNt, uint32_t kThreads>
-__global__ __launch_bounds__(kThreads) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
-  dg_lds_body<kD, kNt, kThreads, false>(a, nullptr);
+template <uint32_t kD, bool kRing, bool kNt>
+__global__ __launch_bounds__(64) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
+  dg_lds_body<kD, kRing, kNt, false, false>(a, nullptr);
 }
-template <bool kNt, uint32_t kThreads>
-__global__ __launch_bounds__(kThreads) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_lds_body<2, kNt, kThreads, true>(a, src);
+template <uint32_t kD, bool kNt, bool kNtStore>
+__global__ __launch_bounds__(64) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
+  dg_lds_body<kD, true, kNt, true, kNtStore>(a, src);
 }
 
 }  // namespace dev
@@ -981,14 +972,19 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * Up to 512 waves, two per CU: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us
 //    against 5.2; 8 MiB 5.3 / 5.7). From about 750 waves the workgroups' 33 KiB of LDS no longer lie evenly over the
 //    CUs (24.8 MB: 7.5 against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
-//  * Up to 80 MB touched: cached loads, in workgroups of one wave. The bytes have just landed, and the engine reads
-//    them next: a non-temporal read of what the caches hold is the slower one (staged 24.8 MB unit, the buffers
-//    changing from pass to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6). Above, whole lines with the
-//    non-temporal hint read faster (336 MiB unit: 55 us against 60; 98.8 MB of odd units 19.0 / 20.4).
+//  * Up to 80 MB touched: two buffers, cached. The bytes have just landed, and the engine reads them next: a
+//    non-temporal read of what the caches hold is the slower one (staged 24.8 MB unit, the buffers changing from pass
+//    to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6).
+//  * Above: four buffers, past the caches (1 and 2 KiB segments). A wave's reads then run through more of a row of
+//    memory at a time: 336 MiB unit 54.9 us, with two buffers 57.3, with eight 55.6, cached 60; 300 MB batch 48.8 /
+//    50.3 / 50.8.
+//    The copy's stores go past the caches from 256 MB on, where they outgrow the last one (199 MB moved 35.0 us
+//    through it, 37.8 past it; 399 MB 77.9 / 71.9).
+constexpr uint64_t kCacheBytes = 256ull << 20;
 enum class Stream { kChain, kAll4, kAll8, kCached, kNt };
 static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
   const bool far = bytes > 80000000;
-  if (seg_bytes % 512 != 0 || seg_bytes > 4096 || (seg_bytes > 2048 && far)) return Stream::kChain;
+  if (seg_bytes % 512 != 0 || seg_bytes > 4096 || (far && seg_bytes != 1024 && seg_bytes != 2048)) return Stream::kChain;
   if (!copy && waves <= 512 && seg_bytes == 2048) return Stream::kAll8;
   if (!copy && waves <= 512 && seg_bytes == 1024) return Stream::kAll4;
   return far ? Stream::kNt : Stream::kCached;
@@ -1015,13 +1011,13 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4) return int(hipErrorInvalidValue);
   const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), a.n * a.unit_bytes, false);
-  const uint32_t threads = rule == Stream::kChain || rule == Stream::kNt ? 256 : 64;
+  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false, 64>
-            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false, 64>
-            : rule == Stream::kCached ? dev::dg_verify_lds_kernel<2, false, 64>
-            : rule == Stream::kNt     ? dev::dg_verify_lds_kernel<2, true, 256>
+  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false, false>
+            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false, false>
+            : rule == Stream::kCached ? dev::dg_verify_lds_kernel<2, true, false>
+            : rule == Stream::kNt     ? dev::dg_verify_lds_kernel<4, true, true>
                                       : dev::dg_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
@@ -1031,12 +1027,14 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
                              hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
-  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), 2 * a.n * a.unit_bytes, true);
-  const uint32_t threads = rule == Stream::kCached ? 64 : 256;
+  const uint64_t bytes = 2 * a.n * a.unit_bytes;
+  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), bytes, true);
+  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<false, 64>
-            : rule == Stream::kNt   ? dev::dg_scatter_verify_lds_kernel<true, 256>
+  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<2, false, false>
+            : rule == Stream::kNt   ? (bytes > kCacheBytes ? dev::dg_scatter_verify_lds_kernel<4, true, true>
+                                                           : dev::dg_scatter_verify_lds_kernel<4, true, false>)
                                     : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
@@ -1047,15 +1045,15 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
                   uint32_t* fail_dev, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (n_units == 0 || n_segments == 0) return 0;
   const Stream rule = stream_rule(seg_bytes, (n_segments + 15) / 16, n_segments * seg_bytes, false);
-  const uint32_t threads = rule == Stream::kChain || rule == Stream::kNt ? 256 : 64;
+  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, 64>
-            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, 64>
-            : rule == Stream::kCached ? dev::verify_kernel<2, false, 64>
-            : rule == Stream::kNt     ? dev::verify_kernel<2, true, 256>
-                                      : dev::verify_kernel<0, false, 256>;
+  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, false, 64>
+            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, false, 64>
+            : rule == Stream::kCached ? dev::verify_kernel<2, true, false, 64>
+            : rule == Stream::kNt     ? dev::verify_kernel<4, true, true, 64>
+                                      : dev::verify_kernel<0, true, false, 256>;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, fail_dev);
 }
