@@ -448,8 +448,8 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
 // segment has whole or not at all is hashed without a select per round: waves at the end of a part are as fast as the
 // others (with both costs in them they were the launch's last: 8 MB in 5.5 us instead of 6.3).
 //
-// What bounds it: reading, from about 50 MB on (336 MiB 55 us, 6.5 TB/s); below, one launch and one to four memory
-// latencies (192 KiB 4.8 us, of which a launch of nothing takes 3.7).
+// What bounds it: reading, from about 50 MB on (336 MiB 55.8 us, 6.4 TB/s); below, one launch and one to four memory
+// latencies (192 KiB 4.9 us, of which a launch of nothing takes 3.7).
 constexpr uint32_t kStateBytes = 1024;  // per wave, at the end of its LDS: 64 bytes per quad
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -532,7 +532,7 @@ __device__ __forceinline__ void drain(F&& hash) {
 // One wave's 16 segments (quad j's lanes 4 j + q hold segment j): where it is read and (kCopy) written, its stripes (0
 // hashes nothing and reads 16 bytes), its checkpoint (32 bytes, 64 when it is not the unit's last). Out: the
 // accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
-// go along with the first live segment and their results mean nothing. The workgroup is one wave, with lds_bytes<kD>().
+// go along with the first live segment and their results mean nothing. lds: the wave's lds_bytes<kD>().
 //
 // kRing: kD chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt
 // 0). Otherwise segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy,
@@ -541,6 +541,10 @@ __device__ __forceinline__ void drain(F&& hash) {
 template <uint32_t kD>
 constexpr uint32_t lds_bytes() {
   return kD * 4096 + kStateBytes;
+}
+template <uint32_t kD>
+__device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
+  return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * lds_bytes<kD>();
 }
 template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
@@ -696,8 +700,8 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
 struct HostSeg {
   const unsigned char* from = nullptr;
   const uint64_t* state = nullptr;
-  uint64_t digest = 0, total = 0;
-  uint32_t stripes = 0, ui = 0;
+  uint64_t digest = 0, total = 0, stripes = 0;
+  uint32_t ui = 0;
   bool live = false, last = false;
   Tail tail;
 };
@@ -725,7 +729,7 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
         const unsigned char* p = static_cast<const unsigned char*>(un.ext[e].ptr);
         const uint64_t off = k * seg_bytes;
         const uint64_t end = off + seg_bytes < span ? off + seg_bytes : span;
-        g.stripes = uint32_t((end - off) / 32);
+        g.stripes = (end - off) / 32;
         g.from = p + off;
         g.last = last_ext && k + 1 == nseg;
         tail = p + span;
@@ -747,11 +751,11 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
 }
 // One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
 // lds_check; 0 runs the chain loop from memory.
-template <uint32_t kD, bool kRing, bool kNt, uint32_t kThreads>
-__global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
-                                                          uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
-                                                          uint32_t* __restrict__ fail) {
-  const uint64_t s0 = (uint64_t(blockIdx.x) * kThreads + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u)) >> 2;
+template <uint32_t kD, bool kRing, bool kNt>
+__global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
+                                                     uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
+                                                     uint32_t* __restrict__ fail) {
+  const uint64_t s0 = (uint64_t(blockIdx.x) * 256 + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u)) >> 2;
   if (s0 >= n_segments) return;  // (the whole wave)
   const uint32_t q = threadIdx.x & 3u;
   const uint64_t s = s0 + ((threadIdx.x & 63u) >> 2);
@@ -772,10 +776,11 @@ __global__ __launch_bounds__(kThreads) void verify_kernel(const TsaVerifyUnit* _
   bool streamed = false;
   if constexpr (kD != 0) {
     streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes<kD>()];  // (one wave)
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
     if (streamed)
-      v = lds_check<kD, kRing, kNt, false, false>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr,
-                                    g.stripes, g.state, g.last, lds, &next);
+      v = lds_check<kD, kRing, kNt, false, false>(
+          g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
+          g.last, wave_lds<kD>(lds), &next);
   }
   if (!streamed && g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -916,8 +921,9 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
 
 template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes<kD>()];
-  const uint64_t gid = uint64_t(blockIdx.x) * 64 + threadIdx.x;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
+  const uint64_t gid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+  if ((gid & ~63ull) >> 2 >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = uint32_t(gid & 3u);
   const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
   Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
@@ -925,7 +931,7 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
     v = lds_check<kD, kRing, kNt, kCopy, kNtStore>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
-                                  g.state, g.last, lds, &next);
+                                  g.state, g.last, wave_lds<kD>(lds), &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
     v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
@@ -933,11 +939,11 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   dg_finish<kCopy>(a, g, tail, v, next, q);
 }
 template <uint32_t kD, bool kRing, bool kNt>
-__global__ __launch_bounds__(64) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
+__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
   dg_lds_body<kD, kRing, kNt, false, false>(a, nullptr);
 }
 template <uint32_t kD, bool kNt, bool kNtStore>
-__global__ __launch_bounds__(64) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
+__global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
   dg_lds_body<kD, true, kNt, true, kNtStore>(a, src);
 }
 
@@ -969,17 +975,17 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * Segments of no whole number of chunk pairs, or longer than 4 KiB: the chain loop (one 24.8 MB unit, 8 KiB segments:
 //    13.1 us; a wave's pieces then lie far apart, and with 4 KiB segments beyond the caches streaming already loses:
 //    122 MB 26.5 us against 23.3).
-//  * Up to 512 waves, two per CU: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us
-//    against 5.2; 8 MiB 5.3 / 5.7). From about 750 waves the workgroups' 33 KiB of LDS no longer lie evenly over the
-//    CUs (24.8 MB: 7.5 against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
+//  * Up to 512 waves: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us against 5.2;
+//    8 MiB 5.3 / 5.7). From about 750 waves its 33 KiB of LDS per wave no longer lie evenly over the CUs (24.8 MB: 7.5
+//    against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
 //  * Up to 80 MB touched: two buffers, cached. The bytes have just landed, and the engine reads them next: a
 //    non-temporal read of what the caches hold is the slower one (staged 24.8 MB unit, the buffers changing from pass
 //    to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6).
 //  * Above: four buffers, past the caches (1 and 2 KiB segments). A wave's reads then run through more of a row of
-//    memory at a time: 336 MiB unit 54.9 us, with two buffers 57.3, with eight 55.6, cached 60; 300 MB batch 48.8 /
-//    50.3 / 50.8.
-//    The copy's stores go past the caches from 256 MB on, where they outgrow the last one (199 MB moved 35.0 us
-//    through it, 37.8 past it; 399 MB 77.9 / 71.9).
+//    memory at a time: 336 MiB unit 56.2 us, with two buffers 57.3, cached 60; 300 MB batch 49.7 / 50.3. The
+//    copy's stores go past the caches from 256 MiB on, where they outgrow the last one (199 MB moved 35.0 us through it,
+//    37.8 past it; 399 MB 77.9 / 71.9).
+// (The figures of the second and third point and of the copy: workgroups of one wave; of four, 1-3 % more.)
 constexpr uint64_t kCacheBytes = 256ull << 20;
 enum class Stream { kChain, kAll4, kAll8, kCached, kNt };
 static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
@@ -1011,7 +1017,7 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4) return int(hipErrorInvalidValue);
   const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), a.n * a.unit_bytes, false);
-  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
+  const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
   auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false, false>
@@ -1029,7 +1035,7 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
   const uint64_t bytes = 2 * a.n * a.unit_bytes;
   const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), bytes, true);
-  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
+  const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
   auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<2, false, false>
@@ -1045,15 +1051,15 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
                   uint32_t* fail_dev, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (n_units == 0 || n_segments == 0) return 0;
   const Stream rule = stream_rule(seg_bytes, (n_segments + 15) / 16, n_segments * seg_bytes, false);
-  const uint32_t threads = rule == Stream::kChain ? 256 : 64;
+  const uint32_t threads = 256;
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, false, 64>
-            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, false, 64>
-            : rule == Stream::kCached ? dev::verify_kernel<2, true, false, 64>
-            : rule == Stream::kNt     ? dev::verify_kernel<4, true, true, 64>
-                                      : dev::verify_kernel<0, true, false, 256>;
+  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, false>
+            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, false>
+            : rule == Stream::kCached ? dev::verify_kernel<2, true, false>
+            : rule == Stream::kNt     ? dev::verify_kernel<4, true, true>
+                                      : dev::verify_kernel<0, true, false>;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, fail_dev);
 }
