@@ -128,13 +128,29 @@ HsaCopier::~HsaCopier() {
 void HsaCopier::wait_all() const {
   std::lock_guard<std::mutex> lk(mu_);
   for (size_t i = 1; i < e_.size(); ++i)
-    for (uint32_t spins = 0; api_->signal_load(e_[i].s) != 0; ++spins) {
+    for (uint32_t spins = 0; !ended_locked(uint32_t(i)); ++spins) {
       if (spins < 4096) _mm_pause();
       else std::this_thread::yield();
     }
 }
 
-bool HsaCopier::done_locked(uint32_t sig) const { return sig == 0 || api_->signal_load(e_[sig].s) == 0; }
+// The runtime sets a failed copy's signal to a negative value. Nothing would ever bring it to 0, which is what the
+// copies that name it wait for: it is set to 0 here, so that they run (into memory the context still holds) and end.
+bool HsaCopier::ended_locked(uint32_t sig) const {
+  if (sig == 0) return true;
+  const hsa_signal_value_t v = api_->signal_load(e_[sig].s);
+  if (v < 0) {
+    failed_ = true;
+    api_->signal_store(e_[sig].s, 0);
+  }
+  return v <= 0;
+}
+
+bool HsaCopier::done_locked(uint32_t sig) const {
+  const bool ended = ended_locked(sig);
+  require(!failed_, SS_E_BACKEND, "HSA: a copy engine reported an error on a unit copy");
+  return ended;
+}
 
 bool HsaCopier::done(uint32_t sig) const {
   if (sig == 0) return true;
@@ -165,7 +181,7 @@ uint32_t HsaCopier::take_locked() {
     std::vector<uint32_t> ended;
     size_t keep = 0;
     for (uint32_t s : retiring_) {
-      if (done_locked(s)) ended.push_back(s);
+      if (ended_locked(s)) ended.push_back(s);
       else retiring_[keep++] = s;
     }
     retiring_.resize(keep);
@@ -194,14 +210,16 @@ uint32_t HsaCopier::take_locked() {
 uint32_t HsaCopier::copy(void* dst, const void* src, uint64_t bytes, bool to_host, const uint32_t* deps,
                          uint32_t n_deps) {
   std::lock_guard<std::mutex> lk(mu_);
+  running_.clear();  // (looked at before a signal is taken: a failed copy throws here)
+  for (uint32_t d = 0; d < n_deps; ++d)
+    if (!done_locked(deps[d])) running_.push_back(deps[d]);
   const uint32_t i = take_locked();
   dep_buf_.clear();
-  for (uint32_t d = 0; d < n_deps; ++d)
-    if (!done_locked(deps[d])) {
-      dep_buf_.push_back(e_[deps[d]].s);
-      ++e_[deps[d]].refs;
-      e_[i].deps.push_back(deps[d]);
-    }
+  for (uint32_t d : running_) {
+    dep_buf_.push_back(e_[d].s);
+    ++e_[d].refs;
+    e_[i].deps.push_back(d);
+  }
   // (the runtime refuses a dependency array with a count of 0 unless it is null)
   const uint32_t nd = uint32_t(dep_buf_.size());
   const hsa_signal_t* dp = nd ? dep_buf_.data() : nullptr;
@@ -222,7 +240,7 @@ bool HsaCopier::copy_ns(uint32_t sig, uint64_t* ns) const {
   if (sig == 0) return false;
   std::lock_guard<std::mutex> lk(mu_);
   hsa_amd_profiling_async_copy_time_t t{};
-  if (!done_locked(sig) || api_->prof_time(e_[sig].s, &t) != HSA_STATUS_SUCCESS || t.end < t.start) return false;
+  if (!ended_locked(sig) || api_->prof_time(e_[sig].s, &t) != HSA_STATUS_SUCCESS || t.end < t.start) return false;
   *ns = uint64_t(double(t.end - t.start) / ticks_per_ns_ + 0.5);
   return true;
 }

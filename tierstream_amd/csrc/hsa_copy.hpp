@@ -33,6 +33,8 @@ class HsaCopier {
   // Signals are indices; 0 is "nothing" (always complete). copy() returns the copy's signal holding one reference
   // (the caller's); a signal goes back to the pool once it has no reference left and its copy has ended.
   // to_host: device memory -> pinned host memory, else the other way. The copy starts once every dep has ended.
+  // A copy whose engine reports an error (a negative signal) counts as ended, the copies behind it run, and done() and
+  // copy() throw from then on: no unit of the context is handed on as landed, and no wait lasts for good.
   uint32_t copy(void* dst, const void* src, uint64_t bytes, bool to_host, const uint32_t* deps, uint32_t n_deps);
   bool done(uint32_t sig) const;
   void ref(uint32_t sig);
@@ -54,14 +56,17 @@ class HsaCopier {
   };
   void release_locked(uint32_t sig);
   uint32_t take_locked();
+  bool ended_locked(uint32_t sig) const;
   bool done_locked(uint32_t sig) const;
 
   const Api* api_;
   hsa_agent_t gpu_{}, cpu_{};
   double ticks_per_ns_ = 1.0;
   mutable std::mutex mu_;
+  mutable bool failed_ = false;        // a copy's engine reported an error
   std::deque<Entry> e_;                // e_[0] unused (index 0 is "nothing")
   std::vector<uint32_t> free_, retiring_;  // free: ended and unreferenced; retiring: unreferenced, maybe running
+  std::vector<uint32_t> running_;      // copy(): its dependencies that have not ended, and their signals
   std::vector<hsa_signal_t> dep_buf_;
 };
 
