@@ -42,6 +42,8 @@ def _fns():
             C.POINTER(C.c_double), C.POINTER(u32)]
     L.tsa_test_depth_ctl.argtypes = args
     L.tsa_test_depth_ctl.restype = C.c_int
+    if not ref.available():
+        return L.tsa_test_depth_ctl, None
     R = ref.lib()
     R.refdg_depth_ctl.argtypes = args
     R.refdg_depth_ctl.restype = C.c_int

@@ -16,6 +16,7 @@ from oracle import fixtures, ref, score_profile
 from tierstream_amd import ss
 
 pytestmark = pytest.mark.gpu
+needs_ref = pytest.mark.skipif(not ref.available(), reason="oracle/_ref not built (needs the reference sources)")
 
 KiB = 1024
 MiB = 1024 * KiB
@@ -197,6 +198,7 @@ HELD = {"scored-profile": "ss_close did not return once after all 24 tokens (120
                           "found by reading, so the case is not run"}
 
 
+@needs_ref
 @pytest.mark.parametrize("name", [pytest.param(n, marks=pytest.mark.skip(reason=HELD[n])) if n in HELD else n
                                   for n in CASES])
 def test_dg_matches_reference(name, tmp_path, gpu):
@@ -492,6 +494,7 @@ RANDOM_THREE_TIER = [
 
 
 # landings: (dg_landing_blocks, dg_landing_ttl, dg_landing_chunk, dg_landing_max_queued)
+@needs_ref
 @pytest.mark.parametrize("clean_evict,queue,parts,predict,bank_keep,adapt,landing",
                          [(0, 0, None, 0, 0, 0, None), (1, 0, None, 0, 0, 0, None), (0, 4, None, 0, 0, 0, None),
                           (1, 4, None, 0, 0, 0, None), (0, 3, BIG_PARTS, 0, 0, 0, None), (0, 4, None, 2, 0, 0, None),
@@ -633,6 +636,7 @@ def test_keep_sched_and_host_calls_refuse_bad_arguments(tmp_path, gpu):
         ctx.close()
 
 
+@needs_ref
 @pytest.mark.parametrize("copies", ["staged", "hsa", "hip"])
 def test_dg_timeline(tmp_path, gpu, copies):
     """dg_diag = 1 (ss_dg_timeline_sized, ss_dg_boundary_timeline_sized; reference ss.h:702-729): after every token each

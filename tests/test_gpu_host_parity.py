@@ -13,6 +13,7 @@ from oracle import fixtures, ref
 from tierstream_amd import ss
 
 pytestmark = pytest.mark.gpu
+needs_ref = pytest.mark.skipif(not ref.available(), reason="oracle/_ref not built (needs the reference sources)")
 
 KiB = 1024
 MiB = 1024 * KiB
@@ -135,6 +136,7 @@ def _stats_doc(text):
     return doc
 
 
+@needs_ref
 @pytest.mark.parametrize("name", list(CASES))
 def test_host_contract_matches_reference(name, tmp_path, gpu):
     ctx, want = _run_case(name, tmp_path, gpu)
@@ -229,6 +231,7 @@ def test_stats_snapshot(name, tmp_path, gpu):
         ctx.close()
 
 
+@needs_ref
 def test_host_prefetch_is_a_checked_no_op_without_read_ahead(tmp_path, gpu):
     """ss_host_prefetch / ss_host_prefetch_layer with readahead_units 0 (reference src/stream_ctx.cpp:1441-1449,
     src/capi.cpp:698-710): a no-op that still refuses a layer out of range and a negative count; the forwards after it
@@ -270,6 +273,7 @@ RA_CASES = {
 }
 
 
+@needs_ref
 @pytest.mark.parametrize("name", list(RA_CASES))
 def test_host_read_ahead_matches_reference(name, tmp_path, gpu):
     """Host read-ahead (readahead_units; reference src/stream_ctx.cpp:212-227, :732-1017, docs/design.md 3.6): file-
