@@ -202,6 +202,12 @@ SS_API ss_status tsa_test_score_profile_check(const void* data, uint64_t len, co
 SS_API uint32_t tsa_test_dgcore_host_order(void* h, uint32_t* out, uint32_t cap);
 /* Landings: per landing block the key it holds (0xFFFFFFFF: none); the return is the landing blocks. */
 SS_API uint32_t tsa_test_dgcore_land_owner(void* h, uint32_t* out, uint32_t cap);
+/* The device-gated service thread over the core alone (no device): started, then stopped as ss_close stops it - where 0 at
+ * once, 1 once it idles, 2 with a token open that no step began, 3 and 4 (a little later) with one that began and whose
+ * first layer never exports. *halted = the outcome it ended with (3: stopped). */
+SS_API ss_status tsa_test_dgcore_service_stop(void* h, uint32_t where, uint32_t* halted);
+/* The watch of a close over three steps, the second of slow_ms: the steps reported as longer than bound_ms, "name;" each. */
+SS_API ss_status tsa_test_close_watch(uint32_t bound_ms, uint32_t slow_ms, char* reports, uint32_t cap);
 SS_API void tsa_test_dgcore_close(void* h);
 
 #ifdef __cplusplus

@@ -2,16 +2,21 @@
 // this library's DgCore on an eager transport, the schedule the reference's CPU tests run its core on
 // (reference tests/test_dg.cpp:201), so placement compares with the reference core's token by token without a GPU.
 #include <algorithm>
+#include <chrono>
+#include <cstdio>
 #include <cstring>
 #include <memory>
 #include <set>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
+#include "close_watch.hpp"
 #include "common.hpp"
 #include "dg_core.hpp"
 #include "depth_ctl.hpp"
+#include "dg_service.hpp"
 #include "score_profile.hpp"
 #include "sha256.hpp"
 #include "tierstream_amd/tsa_test.h"
@@ -342,6 +347,54 @@ uint32_t tsa_test_dgcore_land_owner(void* h, uint32_t* out, uint32_t cap) {
   const std::vector<uint32_t>& v = static_cast<tsa::TestCore*>(h)->core->landing_owners();
   for (uint32_t i = 0; out && i < cap && i < v.size(); ++i) out[i] = v[i];
   return uint32_t(v.size());
+}
+
+ss_status tsa_test_dgcore_service_stop(void* h, uint32_t where, uint32_t* halted) {
+  return tsa::guard([&] {
+    using namespace tsa;
+    require(h && halted && where <= 4, SS_E_INVALID, "tsa_test_dgcore_service_stop: bad argument");
+    DgCore& core = *static_cast<TestCore*>(h)->core;
+    const uint32_t G = core.gated();
+    std::vector<DgRecord> rec(G);
+    std::vector<DgPredRecord> prec(G);
+    std::vector<uint32_t> flag(G, 0), pflag(G, 0);
+    uint32_t words[7] = {};
+    DgMappedHost m;
+    m.rec = rec.data();
+    m.prec = prec.data();
+    m.flag = flag.data();
+    m.pflag = pflag.data();
+    uint32_t** const at[] = {&m.done, &m.err_code, &m.err_aux, &m.err_count, &m.host_abort, &m.host_seq, &m.began};
+    for (int i = 0; i < 7; ++i) *at[i] = words + i;
+    DgService svc(&core, m, kDgMaxIds, 20000, -1);
+    svc.start();
+    const auto nap = [] { std::this_thread::sleep_for(std::chrono::milliseconds(3)); };
+    if (where == 1) nap();  // (past the spin: the idle thread yields)
+    if (where >= 2) svc.begin(1, std::vector<uint8_t>(G, 1));
+    if (where >= 3) {
+      store_release(m.began, 1);
+      if (where == 4) nap();
+    }
+    svc.stop_join();
+    *halted = uint32_t(svc.wait_outcome(1, DgService::Clock::now()));
+  });
+}
+
+ss_status tsa_test_close_watch(uint32_t bound_ms, uint32_t slow_ms, char* reports, uint32_t cap) {
+  return tsa::guard([&] {
+    using namespace tsa;
+    require(reports && cap, SS_E_INVALID, "tsa_test_close_watch: null");
+    std::string got;
+    {
+      CloseWatch w(std::chrono::milliseconds(bound_ms), [&](const char* s, double) { got += std::string(s) + ";"; });
+      const char* const steps[] = {"first", "second", "third"};
+      for (int i = 0; i < 3; ++i) {
+        w.step(steps[i]);
+        std::this_thread::sleep_for(std::chrono::milliseconds(i == 1 ? slow_ms : 0));
+      }
+    }
+    std::snprintf(reports, cap, "%s", got.c_str());
+  });
 }
 
 void tsa_test_dgcore_close(void* h) { delete static_cast<tsa::TestCore*>(h); }

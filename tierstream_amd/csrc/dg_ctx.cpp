@@ -18,6 +18,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "close_watch.hpp"
 #include "dg_core.hpp"
 #include "depth_ctl.hpp"
 #include "dg_geometry.hpp"
@@ -89,13 +90,18 @@ class HipTransport final : public DgTransport {
     }
   }
   ~HipTransport() override {
+    closing("the unit copies issued to the copy engines");
     if (hsa_) hsa_->wait_all();  // every copy out of and into the context's memory has ended
+    closing("the file readers");
     if (pool_) pool_->stop();  // every read's word stored: no await left waiting on the streams below
+    closing("the verify stream");
     if (vs_) (void)hipStreamSynchronize(vs_);
+    closing("the copy streams and their hardware queues");
     for (auto& s : s_) {
       (void)hipStreamSynchronize(s);
       dev_->stream_destroy(s);
     }
+    closing("the transport's memory");
     dev_->free_pinned(stage_host_);
     for (int k = 0; k < 2; ++k) {
       dev_->free_device(stage_dev_[k]);
@@ -103,7 +109,9 @@ class HipTransport final : public DgTransport {
       dev_->free_device(jobs_dev_[k]);
     }
     dev_->free_device(digests_dev_);
+    closing("the verify stream's hardware queue");
     dev_->stream_destroy(vs_);
+    closing("the transport's events and memory");
     for (hipEvent_t e : vev_) dev_->event_destroy(e);
     for (hipEvent_t e : part_ev_) dev_->event_destroy(e);
     dev_->free_pinned(vfail_host_);
@@ -119,6 +127,7 @@ class HipTransport final : public DgTransport {
   }
 
   hipStream_t stream(Stream s) const { return s_[s]; }
+  void set_close_watch(CloseWatch* w) { close_watch_ = w; }
 
   // Unit copies through the HSA runtime (HsaCopier) instead of the HIP streams, possible where every part is copied
   // whole (no scatter) and no file tier reads into the blocks (its reads order the copies behind device waits).
@@ -1019,6 +1028,11 @@ class HipTransport final : public DgTransport {
     pending_.resize(keep);
   }
 
+  void closing(const char* step) {
+    if (close_watch_) close_watch_->step(step);
+  }
+
+  CloseWatch* close_watch_ = nullptr;  // set for the destructor
   std::mutex prof_mu_;  // the service thread brackets demand copies, the engine thread reads and the boundary's copies
   uint32_t prof_mask_ = 0;  // TSA_TEST_PROF_* kinds bracketed
   tsa_test_profile prof_tot_{};
@@ -2287,13 +2301,20 @@ void HipDgCtx::fill() {
 }
 
 void HipDgCtx::release() noexcept {
+  CloseWatch watch;
+  watch.step("the service thread");
   if (svc_) svc_->stop_join();
+  watch.step("the file readers");
   if (tr_) tr_->stop_reads();  // the readers use this context's sources and layout
+  watch.step("the device's work, the engine's streams included");
   if (dev_) (void)hipDeviceSynchronize();
+  watch.step("the cache core");
   svc_.reset();
   core_.reset();
+  if (tr_) tr_->set_close_watch(&watch);
   tr_.reset();
   if (!dev_) return;
+  watch.step("the context's memory");
   for (void* a : arena_) dev_->free_device(a);
   dev_->free_device(slot_of_dev_);
   dev_->free_device(ctl_dev_);

@@ -101,7 +101,7 @@ void DgService::halt(Outcome o, const std::string& why) {
 
 void DgService::thread_main(uint32_t last_seen) {
   try {
-    hip_check(hipSetDevice(device_), "hipSetDevice (service)");
+    if (device_ >= 0) hip_check(hipSetDevice(device_), "hipSetDevice (service)");  // (negative: a test without one)
   } catch (const std::exception& e) {
     halt(Outcome::kFailed, e.what());
     return;
