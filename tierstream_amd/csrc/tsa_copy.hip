@@ -16,10 +16,10 @@ namespace dev {
 // part streams through HBM in order. The job is found by the wave's lanes together and its entry read at once, with
 // scalar loads: block by block, a chain of dependent reads ahead of every 16 KiB cost a tenth of a large launch.
 //
-// kFar (more than 80 MB read and written): nothing of it stays in the caches, and reads and stores go past them. A
-// nearer launch keeps both: the staged bytes have just landed, and the engine reads the slot next. As a copy, source
-// and destination changing from launch to launch, past the caches / through them: 198 MB 63.8 / 68.9 us, 24.8 MB
-// 9.3 / 8.5. Eight units of 24.8 MB 74.4 -> 64.2 us (6.2 TB/s moved), 17 MB in two parts 10.3 -> 7.9.
+// kFar (more than 80 MB read and written): the reads go past the caches. The stores are plain: the engine reads the slot
+// next. Past the caches they were faster only in an unbroken run of launches on changing buffers (396 MB moved: 65.8 us
+// a launch against 73.8); a single launch after other reads took 67.8 against 62.0, one 256 MiB copy on its own 90.4
+// against 79.4.
 constexpr uint32_t kBlock = TSA_SCATTER_BLOCK_BYTES;
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kPerLane = kBlock / (16 * kThreads);  // 4
@@ -61,11 +61,7 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const TsaScatterJob* 
 #pragma unroll
   for (uint32_t k = 0; k < kPerLane; ++k) {
     const uint64_t i = threadIdx.x + uint64_t(k) * kThreads;
-    if (i >= n16) continue;
-    if (kFar)
-      __builtin_nontemporal_store(v[k], d + i);
-    else
-      d[i] = v[k];
+    if (i < n16) d[i] = v[k];
   }
 }
 

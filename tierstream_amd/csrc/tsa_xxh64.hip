@@ -536,8 +536,7 @@ __device__ __forceinline__ void drain(F&& hash) {
 //
 // kRing: kD chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt
 // 0). Otherwise segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy,
-// whose stores the waits would wait for). kNt: reads go past the caches, kNtStore: the
-// copy's stores do.
+// whose stores the waits would wait for). kNt: reads go past the caches.
 template <uint32_t kD>
 constexpr uint32_t lds_bytes() {
   return kD * 4096 + kStateBytes;
@@ -546,7 +545,7 @@ template <uint32_t kD>
 __device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
   return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * lds_bytes<kD>();
 }
-template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
+template <uint32_t kD, bool kRing, bool kNt, bool kCopy>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
                                               uint32_t stripes, const uint64_t* state, bool last,
                                               unsigned char* lds, uint64_t* next) {
@@ -598,11 +597,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     lds_load_chunk<0, kNt>(g, lds_off + buf * 4096);
   };
   auto put = [](unsigned char* p, u32x4 x) {  // (a global store: a generic one would also count on the LDS counter)
-    gu32x4_t* at = reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(p));
-    if (kNtStore)
-      __builtin_nontemporal_store(x, at);
-    else
-      *at = x;
+    *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(p)) = x;
   };
   const bool full = kCopy && __all(live && stripes == 8 * chunks);
   auto store = [&](uint32_t c, uint32_t buf) {  // the lane's own four pieces, as they landed in LDS
@@ -778,7 +773,7 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
     streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
     __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
     if (streamed)
-      v = lds_check<kD, kRing, kNt, false, false>(
+      v = lds_check<kD, kRing, kNt, false>(
           g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
           g.last, wave_lds<kD>(lds), &next);
   }
@@ -919,7 +914,7 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
   dg_chain_body<true>(a, src);
 }
 
-template <uint32_t kD, bool kRing, bool kNt, bool kCopy, bool kNtStore>
+template <uint32_t kD, bool kRing, bool kNt, bool kCopy>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
   const uint64_t gid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -930,7 +925,7 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
-    v = lds_check<kD, kRing, kNt, kCopy, kNtStore>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+    v = lds_check<kD, kRing, kNt, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
                                   g.state, g.last, wave_lds<kD>(lds), &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -940,11 +935,11 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
 }
 template <uint32_t kD, bool kRing, bool kNt>
 __global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
-  dg_lds_body<kD, kRing, kNt, false, false>(a, nullptr);
+  dg_lds_body<kD, kRing, kNt, false>(a, nullptr);
 }
-template <uint32_t kD, bool kNt, bool kNtStore>
+template <uint32_t kD, bool kNt>
 __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_lds_body<kD, true, kNt, true, kNtStore>(a, src);
+  dg_lds_body<kD, true, kNt, true>(a, src);
 }
 
 }  // namespace dev
@@ -983,10 +978,9 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //    to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6).
 //  * Above: four buffers, past the caches (1 and 2 KiB segments). A wave's reads then run through more of a row of
 //    memory at a time: 336 MiB unit 56.2 us, with two buffers 57.3, cached 60; 300 MB batch 49.7 / 50.3. The
-//    copy's stores go past the caches from 256 MiB on, where they outgrow the last one (199 MB moved 35.0 us through it,
-//    37.8 past it; 399 MB 77.9 / 71.9).
+//    copy's stores are plain: past the caches eight staged units (399 MB moved) took 75.2 us against 65.1 after other
+//    reads, and 71.4 against 78.5 only in an unbroken run of launches.
 // (The figures of the second and third point and of the copy: workgroups of one wave; of four, 1-3 % more.)
-constexpr uint64_t kCacheBytes = 256ull << 20;
 enum class Stream { kChain, kAll4, kAll8, kCached, kNt };
 static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
   const bool far = bytes > 80000000;
@@ -1033,14 +1027,12 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
                              hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
-  const uint64_t bytes = 2 * a.n * a.unit_bytes;
-  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), bytes, true);
+  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), 2 * a.n * a.unit_bytes, true);
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<2, false, false>
-            : rule == Stream::kNt   ? (bytes > kCacheBytes ? dev::dg_scatter_verify_lds_kernel<4, true, true>
-                                                           : dev::dg_scatter_verify_lds_kernel<4, true, false>)
+  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<2, false>
+            : rule == Stream::kNt   ? dev::dg_scatter_verify_lds_kernel<4, true>
                                     : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
