@@ -16,15 +16,15 @@ namespace dev {
 // part streams through HBM in order. The job is found by the wave's lanes together and its entry read at once, with
 // scalar loads: block by block, a chain of dependent reads ahead of every 16 KiB cost a tenth of a large launch.
 //
-// kFar (more than 80 MB read and written): the reads go past the caches. The stores are plain: the engine reads the slot
-// next. Past the caches they were faster only in an unbroken run of launches on changing buffers (396 MB moved: 65.8 us
-// a launch against 73.8); a single launch after other reads took 67.8 against 62.0, one 256 MiB copy on its own 90.4
-// against 79.4.
+// Reads go past the caches (each byte is read once), stores do not (the engine reads the slot next). The other ways were
+// faster only in an unbroken run of launches on changing buffers: cached reads 8.9 us against 10.7 for one unit of 24.8
+// MB, non-temporal stores 65.8 against 73.8 for eight. On its own, after a kernel has left the L2 full of written lines,
+// the first takes 17.0 us against 13.0 (the reads drive those lines out); after other reads the second takes 67.8 against
+// 62.0, and a 256 MiB copy 90.4 against 79.4.
 constexpr uint32_t kBlock = TSA_SCATTER_BLOCK_BYTES;
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kPerLane = kBlock / (16 * kThreads);  // 4
 
-template <bool kFar>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(const TsaScatterJob* __restrict__ jobs, uint32_t n_jobs,
                                                            uint64_t n_blocks) {
   const uint64_t blk = blockIdx.x;
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const TsaScatterJob* 
 #pragma unroll
   for (uint32_t k = 0; k < kPerLane; ++k) {
     const uint64_t i = threadIdx.x + uint64_t(k) * kThreads;
-    if (i < n16) v[k] = kFar ? __builtin_nontemporal_load(s + i) : s[i];
+    if (i < n16) v[k] = __builtin_nontemporal_load(s + i);
   }
 #pragma unroll
   for (uint32_t k = 0; k < kPerLane; ++k) {
@@ -183,8 +183,8 @@ __global__ __launch_bounds__(256) void synth_q4_kernel(uint64_t* __restrict__ ds
 int launch_scatter(const TsaScatterJob* jobs_dev, uint32_t n_jobs, uint64_t n_blocks, hipStream_t stream) {
   if (n_jobs == 0 || n_blocks == 0) return 0;
   if (n_blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
-  auto* k = n_blocks * (2 * dev::kBlock) > 80000000 ? dev::scatter_kernel<true> : dev::scatter_kernel<false>;
-  hipLaunchKernelGGL(k, dim3(uint32_t(n_blocks)), dim3(dev::kThreads), 0, stream, jobs_dev, n_jobs, n_blocks);
+  hipLaunchKernelGGL(dev::scatter_kernel, dim3(uint32_t(n_blocks)), dim3(dev::kThreads), 0, stream, jobs_dev, n_jobs,
+                     n_blocks);
   return int(hipGetLastError());
 }
 

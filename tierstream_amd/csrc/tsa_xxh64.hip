@@ -456,67 +456,54 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) u32x4 gu32x4_t;
 
 // M0 (the LDS destination) is restored for the compiler; s_nop: an M0 write before a load to LDS.
-#define TSA_LDS_LOAD16(HINT)                         \
-  asm volatile(                                      \
-      "s_mov_b32 %0, m0\n\t"                         \
-      "s_mov_b32 m0, %2\n\t"                         \
-      "s_nop 0\n\t"                                  \
-      "global_load_lds_dwordx4 %1, off" HINT "\n\t"  \
-      "s_mov_b32 m0, %0\n\t"                         \
-      "s_nop 0"                                      \
-      : "=&s"(save)                                  \
-      : "v"(g), "s"(lds_addr)                        \
-      : "memory")
-template <bool kNt>
 __device__ __forceinline__ void lds_load16(const unsigned char* g, uint32_t lds_addr) {
   uint32_t save;
-  if constexpr (kNt)
-    TSA_LDS_LOAD16(" nt");
-  else
-    TSA_LDS_LOAD16("");
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off nt\n\t"
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0"
+      : "=&s"(save)
+      : "v"(g), "s"(lds_addr)
+      : "memory");
 }
-#undef TSA_LDS_LOAD16
 // A chunk of whole segments: piece k of the lane at g[k] + kAt to lds_addr + 1024 k.
-#define TSA_LDS_LOAD_CHUNK(HINT)                                                                       \
-  asm volatile(                                                                                        \
-      "s_mov_b32 %0, m0\n\t"                                                                           \
-      "s_mov_b32 m0, %5\n\t"                                                                           \
-      "s_nop 0\n\t"                                                                                    \
-      "global_load_lds_dwordx4 %1, off offset:%6" HINT "\n\t"                                          \
-      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
-      "s_nop 0\n\t"                                                                                    \
-      "global_load_lds_dwordx4 %2, off offset:%6" HINT "\n\t"                                          \
-      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
-      "s_nop 0\n\t"                                                                                    \
-      "global_load_lds_dwordx4 %3, off offset:%6" HINT "\n\t"                                          \
-      "s_add_u32 m0, m0, 0x400\n\t"                                                                    \
-      "s_nop 0\n\t"                                                                                    \
-      "global_load_lds_dwordx4 %4, off offset:%6" HINT "\n\t"                                          \
-      "s_mov_b32 m0, %0\n\t"                                                                           \
-      "s_nop 0"                                                                                        \
-      : "=&s"(save)                                                                                    \
-      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr - kAt), "n"(kAt)                      \
-      : "memory", "scc")
-template <uint32_t kAt, bool kNt>
+template <uint32_t kAt>
 __device__ __forceinline__ void lds_load_chunk(const unsigned char* const g[4], uint32_t lds_addr) {
   uint32_t save;
-  if constexpr (kNt)
-    TSA_LDS_LOAD_CHUNK(" nt");
-  else
-    TSA_LDS_LOAD_CHUNK("");
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %5\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off offset:%6 nt\n\t"
+      "s_add_u32 m0, m0, 0x400\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, off offset:%6 nt\n\t"
+      "s_add_u32 m0, m0, 0x400\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %3, off offset:%6 nt\n\t"
+      "s_add_u32 m0, m0, 0x400\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %4, off offset:%6 nt\n\t"
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0"
+      : "=&s"(save)
+      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr - kAt), "n"(kAt)
+      : "memory", "scc");
 }
-#undef TSA_LDS_LOAD_CHUNK
 
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <uint32_t kD, bool kNt, uint32_t kC = 0>
+template <uint32_t kD, uint32_t kC = 0>
 __device__ __forceinline__ void issue_all(const unsigned char* const g[4], uint32_t lds_off) {
   if constexpr (kC < kD) {
-    lds_load_chunk<kC * 256, kNt>(g, lds_off + kC * 4096);
-    issue_all<kD, kNt, kC + 1>(g, lds_off);
+    lds_load_chunk<kC * 256>(g, lds_off + kC * 4096);
+    issue_all<kD, kC + 1>(g, lds_off);
   }
 }
 // Chunk by chunk, each when it has landed (the later ones' loads may still be in flight).
@@ -536,7 +523,7 @@ __device__ __forceinline__ void drain(F&& hash) {
 //
 // kRing: kD chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt
 // 0). Otherwise segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy,
-// whose stores the waits would wait for). kNt: reads go past the caches.
+// whose stores the waits would wait for).
 template <uint32_t kD>
 constexpr uint32_t lds_bytes() {
   return kD * 4096 + kStateBytes;
@@ -545,7 +532,7 @@ template <uint32_t kD>
 __device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
   return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * lds_bytes<kD>();
 }
-template <uint32_t kD, bool kRing, bool kNt, bool kCopy>
+template <uint32_t kD, bool kRing, bool kCopy>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
                                               uint32_t stripes, const uint64_t* state, bool last,
                                               unsigned char* lds, uint64_t* next) {
@@ -569,7 +556,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
   }
   const bool whole = __all(!live || stripes == 8 * chunks);
-  lds_load16<kNt>(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
+  lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
   // The lane's piece of load k (of segment 4k + i: quad 4k + i's lane 0 holds its source) in chunk 0, and how far its
   // segment has later ones: past that the lane loads the last one again, or (no stripe of its own) the segment's first.
   const unsigned char* src[4];
@@ -594,7 +581,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     const unsigned char* g[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) g[k] = src[k] + min(256 * c, lim[k]);
-    lds_load_chunk<0, kNt>(g, lds_off + buf * 4096);
+    lds_load_chunk<0>(g, lds_off + buf * 4096);
   };
   auto put = [](unsigned char* p, u32x4 x) {  // (a global store: a generic one would also count on the LDS counter)
     *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(p)) = x;
@@ -644,7 +631,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
   if constexpr (kRing) {
     auto issue = [&](uint32_t c, uint32_t buf) {
       if (whole) {
-        lds_load_chunk<0, kNt>(src, lds_off + buf * 4096);
+        lds_load_chunk<0>(src, lds_off + buf * 4096);
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) src[k] += 256;
       } else {
@@ -672,7 +659,7 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
     });
   } else {
     if (whole) {
-      issue_all<kD, kNt>(src, lds_off);
+      issue_all<kD>(src, lds_off);
     } else {
 #pragma unroll 1
       for (uint32_t c = 0; c < kD; ++c) issue_part(c, c);
@@ -746,7 +733,7 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
 }
 // One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
 // lds_check; 0 runs the chain loop from memory.
-template <uint32_t kD, bool kRing, bool kNt>
+template <uint32_t kD, bool kRing>
 __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
                                                      uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
                                                      uint32_t* __restrict__ fail) {
@@ -773,7 +760,7 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
     streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
     __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
     if (streamed)
-      v = lds_check<kD, kRing, kNt, false>(
+      v = lds_check<kD, kRing, false>(
           g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
           g.last, wave_lds<kD>(lds), &next);
   }
@@ -914,7 +901,7 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
   dg_chain_body<true>(a, src);
 }
 
-template <uint32_t kD, bool kRing, bool kNt, bool kCopy>
+template <uint32_t kD, bool kRing, bool kCopy>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
   const uint64_t gid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -925,7 +912,7 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
-    v = lds_check<kD, kRing, kNt, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+    v = lds_check<kD, kRing, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
                                   g.state, g.last, wave_lds<kD>(lds), &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -933,13 +920,13 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   }
   dg_finish<kCopy>(a, g, tail, v, next, q);
 }
-template <uint32_t kD, bool kRing, bool kNt>
+template <uint32_t kD, bool kRing>
 __global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
-  dg_lds_body<kD, kRing, kNt, false>(a, nullptr);
+  dg_lds_body<kD, kRing, false>(a, nullptr);
 }
-template <uint32_t kD, bool kNt>
+template <uint32_t kD>
 __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_lds_body<kD, true, kNt, true>(a, src);
+  dg_lds_body<kD, true, true>(a, src);
 }
 
 }  // namespace dev
@@ -973,21 +960,22 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * Up to 512 waves: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us against 5.2;
 //    8 MiB 5.3 / 5.7). From about 750 waves its 33 KiB of LDS per wave no longer lie evenly over the CUs (24.8 MB: 7.5
 //    against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
-//  * Up to 80 MB touched: two buffers, cached. The bytes have just landed, and the engine reads them next: a
-//    non-temporal read of what the caches hold is the slower one (staged 24.8 MB unit, the buffers changing from pass
-//    to pass: 10.3 us against 12.1; 37.6 MB: 17.5 / 22.6).
-//  * Above: four buffers, past the caches (1 and 2 KiB segments). A wave's reads then run through more of a row of
-//    memory at a time: 336 MiB unit 56.2 us, with two buffers 57.3, cached 60; 300 MB batch 49.7 / 50.3. The
-//    copy's stores are plain: past the caches eight staged units (399 MB moved) took 75.2 us against 65.1 after other
-//    reads, and 71.4 against 78.5 only in an unbroken run of launches.
+//  * Up to 80 MB touched: two buffers; above, four (1 and 2 KiB segments): a wave's reads then run through more of a row
+//    of memory at a time: 336 MiB unit 56.2 us, with two buffers 57.3; 300 MB batch 49.7 / 50.3.
+// Every form reads past the caches and (the copy) stores through them, which is what the engine reads next. Cached reads
+// were faster only in an unbroken run of launches on changing buffers (staged 24.8 MB unit 10.2 us against 12.0, 51 MB
+// unit 9.8 / 10.4); after a kernel has left the L2 full of written lines, which cached reads drive out, they took 19.7 us
+// against 15.4 and 23.8 / 13.4, after other reads 15.2 / 15.1 and 14.1 / 13.7, in decode tokens 14.5 / 14.9 and (48 MiB)
+// 13.7 / 13.1. Non-temporal stores: eight staged units (399 MB moved) 75.2 us against 65.1 after other reads, 71.4
+// against 78.5 in an unbroken run.
 // (The figures of the second and third point and of the copy: workgroups of one wave; of four, 1-3 % more.)
-enum class Stream { kChain, kAll4, kAll8, kCached, kNt };
+enum class Stream { kChain, kAll4, kAll8, kRing2, kRing4 };
 static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
   const bool far = bytes > 80000000;
   if (seg_bytes % 512 != 0 || seg_bytes > 4096 || (far && seg_bytes != 1024 && seg_bytes != 2048)) return Stream::kChain;
   if (!copy && waves <= 512 && seg_bytes == 2048) return Stream::kAll8;
   if (!copy && waves <= 512 && seg_bytes == 1024) return Stream::kAll4;
-  return far ? Stream::kNt : Stream::kCached;
+  return far ? Stream::kRing4 : Stream::kRing2;
 }
 
 static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
@@ -1014,10 +1002,10 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false, false>
-            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false, false>
-            : rule == Stream::kCached ? dev::dg_verify_lds_kernel<2, true, false>
-            : rule == Stream::kNt     ? dev::dg_verify_lds_kernel<4, true, true>
+  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false>
+            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false>
+            : rule == Stream::kRing2 ? dev::dg_verify_lds_kernel<2, true>
+            : rule == Stream::kRing4     ? dev::dg_verify_lds_kernel<4, true>
                                       : dev::dg_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
@@ -1031,8 +1019,8 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kCached ? dev::dg_scatter_verify_lds_kernel<2, false>
-            : rule == Stream::kNt   ? dev::dg_scatter_verify_lds_kernel<4, true>
+  auto* k = rule == Stream::kRing2 ? dev::dg_scatter_verify_lds_kernel<2>
+            : rule == Stream::kRing4   ? dev::dg_scatter_verify_lds_kernel<4>
                                     : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
@@ -1047,11 +1035,11 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false, false>
-            : rule == Stream::kAll4   ? dev::verify_kernel<4, false, false>
-            : rule == Stream::kCached ? dev::verify_kernel<2, true, false>
-            : rule == Stream::kNt     ? dev::verify_kernel<4, true, true>
-                                      : dev::verify_kernel<0, true, false>;
+  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false>
+            : rule == Stream::kAll4   ? dev::verify_kernel<4, false>
+            : rule == Stream::kRing2 ? dev::verify_kernel<2, true>
+            : rule == Stream::kRing4     ? dev::verify_kernel<4, true>
+                                      : dev::verify_kernel<0, true>;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, fail_dev);
 }
