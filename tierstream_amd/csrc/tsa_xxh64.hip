@@ -450,7 +450,8 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
 //
 // What bounds it: reading, from about 50 MB on (336 MiB 55.8 us, 6.4 TB/s); below, one launch and one to four memory
 // latencies (192 KiB 4.9 us, of which a launch of nothing takes 3.7).
-constexpr uint32_t kStateBytes = 1024;  // per wave, at the end of its LDS: 64 bytes per quad
+constexpr uint32_t kChunkBuffers = 2 * 4096;              // per wave
+constexpr uint32_t kWaveLds = kChunkBuffers + 64 * 16;  // and 64 bytes of checkpoints per quad behind them
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) u32x4 gu32x4_t;
@@ -469,28 +470,27 @@ __device__ __forceinline__ void lds_load16(const unsigned char* g, uint32_t lds_
       : "v"(g), "s"(lds_addr)
       : "memory");
 }
-// A chunk of whole segments: piece k of the lane at g[k] + kAt to lds_addr + 1024 k.
-template <uint32_t kAt>
+// A chunk: piece k of the lane at g[k] to lds_addr + 1024 k.
 __device__ __forceinline__ void lds_load_chunk(const unsigned char* const g[4], uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %5\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off offset:%6 nt\n\t"
+      "global_load_lds_dwordx4 %1, off nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %2, off offset:%6 nt\n\t"
+      "global_load_lds_dwordx4 %2, off nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %3, off offset:%6 nt\n\t"
+      "global_load_lds_dwordx4 %3, off nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %4, off offset:%6 nt\n\t"
+      "global_load_lds_dwordx4 %4, off nt\n\t"
       "s_mov_b32 m0, %0\n\t"
       "s_nop 0"
       : "=&s"(save)
-      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr - kAt), "n"(kAt)
+      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr)
       : "memory", "scc");
 }
 
@@ -499,40 +499,16 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <uint32_t kD, uint32_t kC = 0>
-__device__ __forceinline__ void issue_all(const unsigned char* const g[4], uint32_t lds_off) {
-  if constexpr (kC < kD) {
-    lds_load_chunk<kC * 256>(g, lds_off + kC * 4096);
-    issue_all<kD, kC + 1>(g, lds_off);
-  }
-}
-// Chunk by chunk, each when it has landed (the later ones' loads may still be in flight).
-template <uint32_t kD, uint32_t kC = 0, class F>
-__device__ __forceinline__ void drain(F&& hash) {
-  if constexpr (kC < kD) {
-    wait_loads<4 * (kD - 1 - kC)>();
-    hash(kC);
-    drain<kD, kC + 1>(hash);
-  }
-}
-
 // One wave's 16 segments (quad j's lanes 4 j + q hold segment j): where it is read and (kCopy) written, its stripes (0
 // hashes nothing and reads 16 bytes), its checkpoint (32 bytes, 64 when it is not the unit's last). Out: the
 // accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
-// go along with the first live segment and their results mean nothing. lds: the wave's lds_bytes<kD>().
+// go along with the first live segment and their results mean nothing. lds: the wave's kWaveLds.
 //
-// kRing: kD chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt
-// 0). Otherwise segments of up to kD chunks, all in flight at once, each hashed when it has landed (not for the copy,
-// whose stores the waits would wait for).
-template <uint32_t kD>
-constexpr uint32_t lds_bytes() {
-  return kD * 4096 + kStateBytes;
-}
-template <uint32_t kD>
+// Two chunk buffers go round: chunk c + 2 is loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0).
 __device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
-  return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * lds_bytes<kD>();
+  return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWaveLds;
 }
-template <uint32_t kD, bool kRing, bool kCopy>
+template <bool kCopy>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
                                               uint32_t stripes, const uint64_t* state, bool last,
                                               unsigned char* lds, uint64_t* next) {
@@ -547,16 +523,12 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
   from = reinterpret_cast<const unsigned char*>(from_first(reinterpret_cast<uintptr_t>(from), reinterpret_cast<uintptr_t>(from)));
   state = reinterpret_cast<const uint64_t*>(from_first(reinterpret_cast<uintptr_t>(state), reinterpret_cast<uintptr_t>(state)));
   last = last || !live;
-  static_assert(kRing || !kCopy, "");
-  uint32_t chunks = kD;
-  if (kRing) {  // as many rounds of the buffers as the wave's longest segment has
-    uint32_t most = stripes;
+  uint32_t most = stripes;  // as many rounds of the buffers as the wave's longest segment has
 #pragma unroll
-    for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
-    chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
-  }
+  for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
+  const uint32_t chunks = max(2u, __builtin_amdgcn_readfirstlane((most + 15) / 16 * 2));
   const bool whole = __all(!live || stripes == 8 * chunks);
-  lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
+  lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kChunkBuffers);
   // The lane's piece of load k (of segment 4k + i: quad 4k + i's lane 0 holds its source) in chunk 0, and how far its
   // segment has later ones: past that the lane loads the last one again, or (no stripe of its own) the segment's first.
   const unsigned char* src[4];
@@ -577,11 +549,17 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
                    __shfl(static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(to)), owner, 64)) +
                at;
   }
-  auto issue_part = [&](uint32_t c, uint32_t buf) {  // not only whole segments
-    const unsigned char* g[4];
+  auto issue = [&](uint32_t c, uint32_t buf) {
+    if (whole) {
+      lds_load_chunk(src, lds_off + buf * 4096);
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) g[k] = src[k] + min(256 * c, lim[k]);
-    lds_load_chunk<0>(g, lds_off + buf * 4096);
+      for (uint32_t k = 0; k < 4; ++k) src[k] += 256;
+    } else {
+      const unsigned char* g[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) g[k] = src[k] + min(256 * c, lim[k]);
+      lds_load_chunk(g, lds_off + buf * 4096);
+    }
   };
   auto put = [](unsigned char* p, u32x4 x) {  // (a global store: a generic one would also count on the LDS counter)
     *reinterpret_cast<gu32x4_t*>(reinterpret_cast<uintptr_t>(p)) = x;
@@ -623,51 +601,29 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
       }
     }
   };
-  auto states = [&] {
-    const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kD * 4096 + j * 64);
-    b = st[q] * P1inv;
-    *next = st[4 + q];
-  };
-  if constexpr (kRing) {
-    auto issue = [&](uint32_t c, uint32_t buf) {
-      if (whole) {
-        lds_load_chunk<0>(src, lds_off + buf * 4096);
+  issue(0, 0);
+  issue(1, 1);
+  wait_loads<8>();
+  const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kChunkBuffers + j * 64);
+  b = st[q] * P1inv;
+  *next = st[4 + q];
+  for (uint32_t c = 0; c + 2 < chunks; c += 2) {
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) src[k] += 256;
-      } else {
-        issue_part(c, buf);
-      }
-    };
-#pragma unroll
-    for (uint32_t c = 0; c < kD; ++c) issue(c, c);
-    wait_loads<4 * kD>();
-    states();
-    for (uint32_t c = 0; c + kD < chunks; c += kD) {
-#pragma unroll
-      for (uint32_t i = 0; i < kD; ++i) {
-        wait_loads<4 * (kD - 1)>();
-        if (kCopy) store(c + i, i);
-        hash(c + i, i);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        issue(c + i + kD, i);
-      }
-    }
-    const uint32_t c = chunks - kD;
-    drain<kD>([&](uint32_t i) {
+    for (uint32_t i = 0; i < 2; ++i) {
+      wait_loads<4>();
       if (kCopy) store(c + i, i);
       hash(c + i, i);
-    });
-  } else {
-    if (whole) {
-      issue_all<kD>(src, lds_off);
-    } else {
-#pragma unroll 1
-      for (uint32_t c = 0; c < kD; ++c) issue_part(c, c);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue(c + i + 2, i);
     }
-    wait_loads<4 * kD>();
-    states();
-    drain<kD>([&](uint32_t c) { hash(c, c); });
   }
+  const uint32_t c = chunks - 2;
+  wait_loads<4>();
+  if (kCopy) store(c, 0);
+  hash(c, 0);
+  wait_loads<0>();
+  if (kCopy) store(c + 1, 1);
+  hash(c + 1, 1);
   return b * P1;
 }
 
@@ -731,9 +687,9 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
   g.total = un.total;
   return g;
 }
-// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
-// lds_check; 0 runs the chain loop from memory.
-template <uint32_t kD, bool kRing>
+// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kStream:
+// waves of 16-byte aligned segments stream through LDS; any other runs the chain loop from memory.
+template <bool kStream>
 __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
                                                      uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
                                                      uint32_t* __restrict__ fail) {
@@ -756,13 +712,13 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
   if (__ballot(g.live) == 0) return;
   uint64_t v = 0, next = 0;
   bool streamed = false;
-  if constexpr (kD != 0) {
+  if constexpr (kStream) {
     streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
     if (streamed)
-      v = lds_check<kD, kRing, false>(
+      v = lds_check<false>(
           g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
-          g.last, wave_lds<kD>(lds), &next);
+          g.last, wave_lds(lds), &next);
   }
   if (!streamed && g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -901,9 +857,9 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
   dg_chain_body<true>(a, src);
 }
 
-template <uint32_t kD, bool kRing, bool kCopy>
+template <bool kCopy>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * lds_bytes<kD>()];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
   const uint64_t gid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
   if ((gid & ~63ull) >> 2 >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = uint32_t(gid & 3u);
@@ -912,21 +868,17 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
-    v = lds_check<kD, kRing, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
-                                  g.state, g.last, wave_lds<kD>(lds), &next);
+    v = lds_check<kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+                                  g.state, g.last, wave_lds(lds), &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
     v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
   }
   dg_finish<kCopy>(a, g, tail, v, next, q);
 }
-template <uint32_t kD, bool kRing>
-__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) {
-  dg_lds_body<kD, kRing, false>(a, nullptr);
-}
-template <uint32_t kD>
+__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) { dg_lds_body<false>(a, nullptr); }
 __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_lds_body<kD, true, true>(a, src);
+  dg_lds_body<true>(a, src);
 }
 
 }  // namespace dev
@@ -953,29 +905,23 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
   return int(hipGetLastError());
 }
 
-// How a launch of `waves` waves of 16 segments that touches `bytes` (the copy: twice its units') runs.
-//  * Segments of no whole number of chunk pairs, or longer than 4 KiB: the chain loop (one 24.8 MB unit, 8 KiB segments:
-//    13.1 us; a wave's pieces then lie far apart, and with 4 KiB segments beyond the caches streaming already loses:
-//    122 MB 26.5 us against 23.3).
-//  * Up to 512 waves: every chunk in flight at once, one memory latency instead of four (192 KiB: 4.9 us against 5.2;
-//    8 MiB 5.3 / 5.7). From about 750 waves its 33 KiB of LDS per wave no longer lie evenly over the CUs (24.8 MB: 7.5
-//    against 6.9). The copy gains nothing from it (11.4 against 10.8 for one 24.8 MB unit).
-//  * Up to 80 MB touched: two buffers; above, four (1 and 2 KiB segments): a wave's reads then run through more of a row
-//    of memory at a time: 336 MiB unit 56.2 us, with two buffers 57.3; 300 MB batch 49.7 / 50.3.
-// Every form reads past the caches and (the copy) stores through them, which is what the engine reads next. Cached reads
-// were faster only in an unbroken run of launches on changing buffers (staged 24.8 MB unit 10.2 us against 12.0, 51 MB
-// unit 9.8 / 10.4); after a kernel has left the L2 full of written lines, which cached reads drive out, they took 19.7 us
-// against 15.4 and 23.8 / 13.4, after other reads 15.2 / 15.1 and 14.1 / 13.7, in decode tokens 14.5 / 14.9 and (48 MiB)
-// 13.7 / 13.1. Non-temporal stores: eight staged units (399 MB moved) 75.2 us against 65.1 after other reads, 71.4
-// against 78.5 in an unbroken run.
-// (The figures of the second and third point and of the copy: workgroups of one wave; of four, 1-3 % more.)
-enum class Stream { kChain, kAll4, kAll8, kRing2, kRing4 };
-static Stream stream_rule(uint64_t seg_bytes, uint64_t waves, uint64_t bytes, bool copy) {
-  const bool far = bytes > 80000000;
-  if (seg_bytes % 512 != 0 || seg_bytes > 4096 || (far && seg_bytes != 1024 && seg_bytes != 2048)) return Stream::kChain;
-  if (!copy && waves <= 512 && seg_bytes == 2048) return Stream::kAll8;
-  if (!copy && waves <= 512 && seg_bytes == 1024) return Stream::kAll4;
-  return far ? Stream::kRing4 : Stream::kRing2;
+// Whether a launch that touches `bytes` (the copy: twice its units') streams its segments. Not segments of no whole
+// number of chunk pairs, or longer than 4 KiB (one 24.8 MB unit, 8 KiB segments: 13.1 us; a wave's pieces then lie far
+// apart, and with 4 KiB segments beyond the caches streaming already loses: 122 MB 26.5 us against 23.3).
+//
+// One form for all sizes: two buffers a wave, reads past the caches, stores (the copy's) through them. Tried against it,
+// in workgroups of four waves, us (in a loop on changing buffers / one launch after other reads):
+//  * Four buffers (70 KB of LDS a workgroup, two on a CU): 85 MB 16.0 / 19.9, two 15.5 / 19.0; 300 MB batch 48.4 / 53.0,
+//    two 47.8 / 50.6; with 1 KiB segments 54.5 / 59.0, two 50.0 / 52.1.
+//  * All of a segment's chunks in flight at once (132 KiB a workgroup): 64 waves 5.53 / 9.16, ring 5.44 / 9.04; 512 waves
+//    6.68 / 9.56, ring 6.58 / 9.44. Better only for a single wave (5.0 / 8.3, ring 5.1 / 9.2).
+//  * Cached reads, faster only in the loop (staged 24.8 MB unit 10.2 us against 12.0, 51 MB unit 9.8 / 10.4): after a
+//    kernel has left the L2 full of written lines, which they drive out, 19.7 us against 15.4 and 23.8 against 13.4; in
+//    decode tokens 14.5 against 14.9 and (48 MiB) 13.7 against 13.1.
+//  * Non-temporal stores, likewise: eight staged units (399 MB moved) 71.4 us against 78.5 in the loop, 75.2 against 65.1
+//    after other reads.
+static bool streams(uint64_t seg_bytes, uint64_t bytes) {
+  return seg_bytes % 512 == 0 && seg_bytes <= 4096 && (bytes <= 80000000 || seg_bytes == 1024 || seg_bytes == 2048);
 }
 
 static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
@@ -998,15 +944,10 @@ static int launch_timed(K* k, dim3 grid, uint32_t threads, hipStream_t stream, h
 int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4) return int(hipErrorInvalidValue);
-  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), a.n * a.unit_bytes, false);
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kAll8     ? dev::dg_verify_lds_kernel<8, false>
-            : rule == Stream::kAll4   ? dev::dg_verify_lds_kernel<4, false>
-            : rule == Stream::kRing2 ? dev::dg_verify_lds_kernel<2, true>
-            : rule == Stream::kRing4     ? dev::dg_verify_lds_kernel<4, true>
-                                      : dev::dg_verify_kernel;
+  auto* k = streams(a.seg_bytes, a.n * a.unit_bytes) ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
 }
@@ -1015,13 +956,10 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
                              hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
-  const Stream rule = stream_rule(a.seg_bytes, a.n * ((a.unit_segs + 15) / 16), 2 * a.n * a.unit_bytes, true);
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = rule == Stream::kRing2 ? dev::dg_scatter_verify_lds_kernel<2>
-            : rule == Stream::kRing4   ? dev::dg_scatter_verify_lds_kernel<4>
-                                    : dev::dg_scatter_verify_kernel;
+  auto* k = streams(a.seg_bytes, 2 * a.n * a.unit_bytes) ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
@@ -1030,16 +968,11 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
 int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_segments, uint64_t seg_bytes,
                   uint32_t* fail_dev, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (n_units == 0 || n_segments == 0) return 0;
-  const Stream rule = stream_rule(seg_bytes, (n_segments + 15) / 16, n_segments * seg_bytes, false);
   const uint32_t threads = 256;
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = rule == Stream::kAll8     ? dev::verify_kernel<8, false>
-            : rule == Stream::kAll4   ? dev::verify_kernel<4, false>
-            : rule == Stream::kRing2 ? dev::verify_kernel<2, true>
-            : rule == Stream::kRing4     ? dev::verify_kernel<4, true>
-                                      : dev::verify_kernel<0, true>;
+  auto* k = streams(seg_bytes, n_segments * seg_bytes) ? dev::verify_kernel<true> : dev::verify_kernel<false>;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, fail_dev);
 }
