@@ -704,10 +704,24 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
   const TsaVerifyUnit un = units[ui];  // (whole and at once: with scalar loads, one memory latency)
   if (after >= end) {
     if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
-  } else if (s < end) {
-    while (ui + 1 < n_units && units[ui + 1].seg_first <= s) ++ui;
-    const TsaVerifyUnit mine = units[ui];
-    g = host_segment(mine, ui, s, seg_bytes, shift, fail, q);
+  } else {
+    // The quad's unit: the next 16 units' first segments in one read, counted up to the quad's own (unit by unit, 200
+    // units of one segment each were 16 reads one behind the other: 8.6 us, 7.2 like this).
+    const uint64_t base = ui + 1;
+    for (uint64_t w = base, seen = after; seen < end; w += 16) {
+      const uint64_t i = w + (threadIdx.x & 15u);
+      const uint64_t f = i < n_units ? units[i].seg_first : ~0ull;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        seen = uint64_t(uint32_t(__builtin_amdgcn_readlane(int(f >> 32), k))) << 32 |
+               uint32_t(__builtin_amdgcn_readlane(int(f), k));
+        ui += seen <= s;
+      }
+    }
+    if (s < end) {
+      const TsaVerifyUnit mine = units[ui];
+      g = host_segment(mine, ui, s, seg_bytes, shift, fail, q);
+    }
   }
   if (__ballot(g.live) == 0) return;
   uint64_t v = 0, next = 0;
