@@ -919,9 +919,11 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
   return int(hipGetLastError());
 }
 
-// Whether a launch that touches `bytes` (the copy: twice its units') streams its segments. Not segments of no whole
-// number of chunk pairs, or longer than 4 KiB (one 24.8 MB unit, 8 KiB segments: 13.1 us; a wave's pieces then lie far
-// apart, and with 4 KiB segments beyond the caches streaming already loses: 122 MB 26.5 us against 23.3).
+// Whether a launch streams its segments: a check those of 1 and 2 KiB, the copy (which touches `bytes`, twice its units')
+// also others of whole chunk pairs, up to 4 KiB and 80 MB. Checks, streamed / chain loop, us in a loop on changing buffers:
+// 8.6 MB in 1.5 KiB segments 5.4 / 4.5, 8.4 MB in 4 KiB segments 7.9 / 6.4, 62 MB in 512-byte ones 11.9 / 10.9 (a wave's
+// pieces lie far apart, or a wave ends after one pair). The copy: 17 MB moved in 4 KiB segments 11.4 / 13.8, in 1.5 KiB
+// ones 7.7 / 8.0.
 //
 // One form for all sizes: two buffers a wave, reads past the caches, stores (the copy's) through them. Tried against it,
 // in workgroups of four waves, us (in a loop on changing buffers / one launch after other reads):
@@ -934,8 +936,22 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //    decode tokens 14.5 against 14.9 and (48 MiB) 13.7 against 13.1.
 //  * Non-temporal stores, likewise: eight staged units (399 MB moved) 71.4 us against 78.5 in the loop, 75.2 against 65.1
 //    after other reads.
-static bool streams(uint64_t seg_bytes, uint64_t bytes) {
-  return seg_bytes % 512 == 0 && seg_bytes <= 4096 && (bytes <= 80000000 || seg_bytes == 1024 || seg_bytes == 2048);
+constexpr uint64_t kNearBytes = 80000000;
+static bool check_streams(uint64_t seg_bytes) { return seg_bytes == 1024 || seg_bytes == 2048; }
+static bool copy_streams(uint64_t seg_bytes, uint64_t bytes) {
+  return check_streams(seg_bytes) || (seg_bytes % 512 == 0 && seg_bytes <= 4096 && bytes <= kNearBytes);
+}
+// Whether every part of every unit of the launch lies 16-byte aligned. One that does not streams wave by wave only above
+// 80 MB (102 MB, a third of it unaligned: 16.0 us against 18.9 for the chain loop on the same buffers); below, the chain
+// loop's kernel with its 8 waves on a SIMD is the better one (8.5 MB 5.2 us, wave by wave 5.8; 34 MB 7.7 / 7.9).
+static bool aligned16(const DgVerifyLaunch& a) {
+  for (uint32_t p = 0; p < a.n_parts; ++p) {
+    if (reinterpret_cast<uintptr_t>(a.arena[p]) % 16 != 0) return false;
+    if (a.part_bytes[p] % 16 == 0) continue;
+    for (uint32_t u = 0; u < a.n; ++u)
+      if (uint64_t(a.slots[u]) * a.part_bytes[p] % 16 != 0) return false;
+  }
+  return true;
 }
 
 static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
@@ -961,7 +977,8 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = streams(a.seg_bytes, a.n * a.unit_bytes) ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
+  const bool stream_it = check_streams(a.seg_bytes) && (a.n * a.unit_bytes > kNearBytes || aligned16(a));
+  auto* k = stream_it ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
 }
@@ -973,7 +990,7 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = streams(a.seg_bytes, 2 * a.n * a.unit_bytes) ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
+  auto* k = copy_streams(a.seg_bytes, 2 * a.n * a.unit_bytes) ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
@@ -986,7 +1003,7 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = streams(seg_bytes, n_segments * seg_bytes) ? dev::verify_kernel<true> : dev::verify_kernel<false>;
+  auto* k = check_streams(seg_bytes) ? dev::verify_kernel<true> : dev::verify_kernel<false>;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, fail_dev);
 }
