@@ -29,6 +29,24 @@ def test_digest_unit_counts(gpu, n):
     assert gpu.device_digests(units) == want
 
 
+# Workgroups whose units all have at most 32 stripes hash them straight from memory; one with a stripe more is fed.
+@pytest.mark.parametrize("n", [2, 513, 1025, 2049, 4097, 12288])
+@pytest.mark.parametrize("longest", [1024 + 31, 1024 + 32])
+def test_digest_small_units(gpu, n, longest):
+    rng = np.random.default_rng(n)
+    data = rng.integers(0, 256, 1 << 16, dtype=np.uint8)
+    buf = gpu.DeviceBuffer(data.nbytes)
+    buf.upload(data)
+    shapes = [[0], [7], [32], [1023], [32, 0], [512, 512], [96, 64, 32, 33], [longest], [512, 32, longest - 544]]
+    units, want = [], []
+    for i in range(n):
+        sizes = shapes[(i + i // 9) % len(shapes)] if i % 64 < 48 else [64]  # (long ones in some workgroups only)
+        at = [int(rng.integers((data.nbytes - s) // 8)) * 8 for s in sizes]
+        units.append(gpu.make_unit([(buf.ptr + a, s) for a, s in zip(at, sizes)]))
+        want.append(xxhash.xxh64_intdigest(b"".join(data[a:a + s].tobytes() for a, s in zip(at, sizes))))
+    assert gpu.device_digests(units) == want
+
+
 # Kind 2 is made in groups of nine words (four Q4 blocks), 256 groups to a workgroup; kinds 0 and 1 two words to a lane.
 @pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("words,offset", [(1, 0), (2, 1), (8, 8), (9, 9), (511, 3), (2304, 0), (2304, 5), (2305, 2300),

@@ -217,6 +217,10 @@ constexpr uint32_t kFeeders = 256;       // feeding lanes (four waves)
 constexpr uint32_t kFeedStripes = 512;   // stripes of a chunk, all units of the workgroup
 constexpr uint32_t kFeedLoads = kFeedStripes * 2 / kFeeders;  // 16-byte pieces per lane and chunk
 constexpr uint32_t kHashAhead = 16;      // stripes the hashing wave holds in registers ahead
+// A workgroup whose units have no more than this many stripes hashes them quad by quad from memory: one 64-byte unit 6.7
+// us, fed 8.2; 512 units of 512 bytes 7.8 / 9.5; 12288 of 1 KiB 9.3 / 12.1. At 2 KiB feeding is even with it (7.6 / 8.5,
+// after other reads 9.8 / 9.4).
+constexpr uint32_t kDirect = 32;
 
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
@@ -227,6 +231,8 @@ struct UnitStripes {
   uintptr_t base[TSA_MAX_EXTENTS];
   uint64_t end[TSA_MAX_EXTENTS];
   uint64_t bytes;
+  const unsigned char* tail;  // the bytes after the last stripe
+  uint32_t tail_len;
 };
 
 // kHashAhead rounds on the products r, from the state b to the state b (see above). Written out because its speed hangs
@@ -274,17 +280,26 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
   const uint32_t u = blockIdx.x * kG + mine;
   if (tid < kG) {
     const uint32_t v = blockIdx.x * kG + tid;
-    const uint32_t ext = v < n ? units[v].n_ext : 0;
+    const TsaUnit un = units[v < n ? v : n - 1];  // (whole: one memory latency)
+    const uint32_t ext = v < n ? un.n_ext : 0;
     uint64_t at = 0, sum = 0;
+    const unsigned char* tail = nullptr;
+    uint32_t tail_len = 0;
 #pragma unroll
     for (uint32_t e = 0; e < TSA_MAX_EXTENTS; ++e) {
-      const uint64_t bytes = e < ext ? units[v].ext[e].bytes : 0;
-      table[tid].base[e] = (e < ext ? reinterpret_cast<uintptr_t>(units[v].ext[e].ptr) : 0) - 32 * at;
+      const uint64_t bytes = e < ext ? un.ext[e].bytes : 0;
+      table[tid].base[e] = (e < ext ? reinterpret_cast<uintptr_t>(un.ext[e].ptr) : 0) - 32 * at;
       at += bytes / 32;
       table[tid].end[e] = at;
       sum += bytes;
+      if (e < ext) {
+        tail = static_cast<const unsigned char*>(un.ext[e].ptr) + bytes / 32 * 32;
+        tail_len = uint32_t(bytes % 32);
+      }
     }
     table[tid].bytes = sum;
+    table[tid].tail = tail;
+    table[tid].tail_len = tail_len;
   }
   __syncthreads();
   const UnitStripes& us = table[mine];
@@ -299,6 +314,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
                           __builtin_amdgcn_readfirstlane(uint32_t((most + kC - 1) / kC));
 
   if (feeds) {
+    if (most <= kDirect) return;
     constexpr uint32_t kLanes = kFeeders / kG;  // of one unit: lane l moves half l & 1 of stripes l / 2 + j kLanes / 2
     const uint32_t l = (tid - 64) % kLanes;
     unsigned char* row = lds + (4 * mine + (l & 1u) * 2) * kRow + (l >> 1) * 8;
@@ -359,8 +375,25 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
     return;
   }
 
-  __builtin_amdgcn_s_setprio(3);
   const uint32_t q = tid & 3u;
+  const bool ends = tid < 4 * kG && q == 0 && u < n;
+  Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
+  if (ends) tail = load_tail(us.tail, us.tail_len);
+  if (most <= kDirect) {  // (the feeders have ended)
+    uint64_t acc[4];
+    init_acc(acc);
+    uint64_t v = q == 0 ? acc[0] : q == 1 ? acc[1] : q == 2 ? acc[2] : acc[3], at = 0;
+    for (uint32_t e = 0; e < TSA_MAX_EXTENTS && at < total; ++e) {
+      v = chain(v, reinterpret_cast<const unsigned char*>(us.base[e] + 32 * at), us.end[e] - at, q);
+      at = us.end[e];
+    }
+    uint64_t all[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int((tid & ~3u) + k), 64);
+    if (ends) out[u] = xfinal(all, us.bytes, tail);
+    return;
+  }
+  __builtin_amdgcn_s_setprio(3);
   const unsigned char* row = lds + (4 * mine + q) * kRow;
   uint64_t acc[4];
   init_acc(acc);
@@ -413,17 +446,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
   uint64_t all[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) all[k] = __shfl(v, int((tid & ~3u) + k), 64);
-  if (tid < 4 * kG && q == 0 && u < n) {
-    const uint32_t ext = units[u].n_ext < TSA_MAX_EXTENTS ? units[u].n_ext : TSA_MAX_EXTENTS;
-    const unsigned char* tail = nullptr;
-    uint32_t tail_len = 0;
-    if (ext) {
-      const uint64_t bytes = units[u].ext[ext - 1].bytes;
-      tail = static_cast<const unsigned char*>(units[u].ext[ext - 1].ptr) + bytes / 32 * 32;
-      tail_len = uint32_t(bytes % 32);
-    }
-    out[u] = xfinal(all, us.bytes, load_tail(tail, tail_len));
-  }
+  if (ends) out[u] = xfinal(all, us.bytes, tail);
 }
 
 // ---- The LDS-streamed check (segments of a multiple of 512 bytes) ----
