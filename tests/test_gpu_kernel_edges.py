@@ -77,16 +77,17 @@ def test_synth_edges(gpu, kind, words, offset):
             assert np.array_equal(got, synth.uniform_bytes(99, 5, at, n) if kind == 0 else synth.q4_blocks(99, 5, at, n))
 
 
-# The checks by segment size and by size: all chunks of a wave in flight (1 and 2 KiB segments, up to 512 waves), two
-# chunk buffers (whole pairs of 256-byte chunks), four with non-temporal reads (above 80 MB; non-temporal stores too
-# above 256 MiB moved), the chain loop (other segments; waves with a segment that is 8-byte aligned); parts that end
-# inside a segment, inside a stripe, or are none.
+# The checks by segment size and by size: two chunk buffers a wave (1 and 2 KiB segments, any whole pair of 256-byte chunks
+# in the copy up to 80 MB), the chain loop (other segments; up to 80 MB also arenas with a part that is 8-byte aligned;
+# above, and in batches and the copy, the waves that hold one); parts that end inside a segment, inside a stripe, or are
+# none.
 SHAPES = [
     (1, [2048], 2048), (1, [32], 2048), (2, [8], 2048), (1, [2080, 40], 2048), (5, [65568, 4096, 1000], 2048),
     (64, [30 * 2048 + 32, 96], 2048), (3, [2048 * 17, 2048 * 15 + 64, 32, 2048], 2048), (3, [(8 << 20) + 32, 1 << 20], 2048),
     (3, [28 << 20, (3 << 20) + 48], 2048), (3, [45 << 20, 4096 + 24], 2048), (2, [65536, 2048 + 1008], 512), (3, [65536 + 96, 1024 * 16], 1024),
     (2, [9 << 20, 1024 * 3 + 8], 1024), (3, [1536 * 40 + 32, 1536 * 16 - 8], 1536), (2, [1 << 20, 4096 * 3 + 56], 4096),
-    (3, [28 << 20, 4096 + 16], 4096), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
+    (3, [28 << 20, 4096 + 16], 4096), (3, [28 << 20, (3 << 20) + 1000], 1024),
+    (3, [44 << 20, (3 << 20) + 48], 1024), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
 ]
 
 
@@ -187,7 +188,56 @@ def test_batch_checks_by_shape(gpu, n, parts, seg, align):
         assert list(fail.download(4 * n).view(np.uint32)) == want
 
 
-# 16 KiB blocks part by part; more jobs than a wave's 64 probes; near (cached) and, above 80 MB moved, far launches.
+# A checkpoint is four 64-bit words: it may lie 8-byte aligned, and the kernels read it in 16-byte pieces.
+@pytest.mark.parametrize("how", ["check", "staged", "batch"])
+@pytest.mark.parametrize("parts,seg", [([65536 + 96, 4000], 2048), ([65536, 1024 * 3 + 8], 1024), ([32768 + 32, 40], 4096)])
+def test_checkpoints_at_8_bytes(gpu, how, parts, seg):
+    rng = np.random.default_rng(seg)
+    n, ub = 3, sum(parts)
+    data = rng.integers(0, 256, (n, ub), dtype=np.uint8)
+    cuts = np.cumsum([0] + parts)
+    marks = [gpu.host_checkpoints([u[a:b] for a, b in zip(cuts, cuts[1:])], seg) for u in data]
+    words = len(marks[0][0])
+    st_dev, fail = gpu.DeviceBuffer(8 + 8 * words * n), gpu.DeviceBuffer(4 * n)
+    st_dev.upload(np.concatenate([np.zeros(1, dtype=np.uint64)] + [st for st, _ in marks]))
+    states = st_dev.ptr + 8
+    assert states % 16 == 8
+    src = gpu.DeviceBuffer(n * ub)
+    for bad in (None, 1):
+        if bad is not None:
+            data[bad, parts[0] - 1] ^= 1
+        src.upload(data.reshape(-1))
+        fail.upload(np.zeros(n, dtype=np.uint32))
+        if how == "batch":
+            units = []
+            for i in range(n):
+                v = gpu.TsaVerifyUnit()
+                for e, (at, b) in enumerate(zip(cuts, parts)):
+                    v.ext[e].ptr, v.ext[e].bytes = src.ptr + i * ub + int(at), b
+                v.n_ext, v.seg_first, v.digest, v.total = len(parts), i * words // 4, marks[i][1], ub
+                v.states = states + 8 * words * i
+                units.append(v)
+            table = gpu.upload_struct_array(units)
+            gpu.check(gpu.lib().tsa_xxh64_verify(C.c_void_p(table.ptr), n, n * words // 4, seg, C.c_void_p(fail.ptr), None))
+        else:
+            dg_dev = gpu.DeviceBuffer(8 * n)
+            dg_dev.upload(np.array([dg for _, dg in marks], dtype=np.uint64))
+            bufs = [gpu.DeviceBuffer(n * p) for p in parts]
+            a = gpu.TsaArenaVerify()
+            for p, (buf, pb) in enumerate(zip(bufs, parts)):
+                buf.upload(np.ascontiguousarray(data[:, cuts[p]:cuts[p + 1]]).reshape(-1))
+                a.arena[p], a.part_bytes[p] = buf.ptr, pb
+            a.n_parts, a.seg_bytes, a.states_dev, a.digests_dev = len(parts), seg, states, dg_dev.ptr
+            args = [C.byref(a), (C.c_uint32 * n)(*range(n)), (C.c_int32 * n)(*range(n)), n]
+            if how == "staged":
+                gpu.check(gpu.lib().tsa_xxh64_scatter_verify_slots(*args, C.c_void_p(src.ptr), C.c_void_p(fail.ptr), None))
+            else:
+                gpu.check(gpu.lib().tsa_xxh64_verify_slots(*args, C.c_void_p(fail.ptr), None))
+        gpu.check(gpu.lib().tsa_stream_sync(None))
+        assert list(fail.download(4 * n).view(np.uint32)) == [int(i == bad) for i in range(n)]
+
+
+# 16 KiB blocks part by part; more jobs than a wave's 64 probes.
 @pytest.mark.parametrize("n,parts", [(1, [16]), (1, [16384]), (2, [16400, 32, 0, 16368]), (65, [16384 * 3, 48]),
                                      (200, [1024, 16]), (3, [13 << 20, (1 << 20) + 16])])
 def test_scatter_jobs(gpu, n, parts):
