@@ -758,8 +758,10 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
           g.last, wave_lds(lds), &next);
   }
   if (!streamed && g.live) {
-    next = g.last ? 0 : g.state[4 + q];
-    v = chain_t<false>(g.state[q], g.from, nullptr, g.stripes, q);
+    // (global loads: with a generic one under way the compiler waits for all of a block's words before its first round)
+    gword_t* const state = reinterpret_cast<gword_t*>(reinterpret_cast<uintptr_t>(g.state));
+    next = g.last ? 0 : state[4 + q];
+    v = chain(state[q], g.from, g.stripes, q);
   }
   uint64_t all[4];
   const uint32_t base = threadIdx.x & ~3u;
