@@ -710,12 +710,12 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
   g.total = un.total;
   return g;
 }
-// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kStream:
-// waves of 16-byte aligned segments stream through LDS; any other runs the chain loop from memory.
-template <bool kStream>
-__global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
-                                                     uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
-                                                     uint32_t* __restrict__ fail) {
+// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kLds: waves
+// whose segments all start at a multiple of `mask` + 1 stream through LDS; any other runs the chain loop from memory.
+template <bool kLds>
+__device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ units, uint32_t n_units, uint64_t n_segments,
+                                            uint64_t seg_bytes, uint32_t shift, uint64_t mask,
+                                            uint32_t* __restrict__ fail) {
   const uint64_t s0 = (uint64_t(blockIdx.x) * 256 + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u)) >> 2;
   if (s0 >= n_segments) return;  // (the whole wave)
   const uint32_t q = threadIdx.x & 3u;
@@ -749,8 +749,8 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
   if (__ballot(g.live) == 0) return;
   uint64_t v = 0, next = 0;
   bool streamed = false;
-  if constexpr (kStream) {
-    streamed = __all(!g.live || reinterpret_cast<uintptr_t>(g.from) % 16 == 0);
+  if constexpr (kLds) {
+    streamed = __all(!g.live || (reinterpret_cast<uintptr_t>(g.from) & mask) == 0);
     __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
     if (streamed)
       v = lds_check<false>(
@@ -773,6 +773,16 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
   } else if (q == 0) {
     if (xfinal(all, g.total, g.tail) != g.digest) atomicOr(fail + g.ui, 1u);
   }
+}
+__global__ __launch_bounds__(256) void verify_lds_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
+                                                         uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
+                                                         uint64_t mask, uint32_t* __restrict__ fail) {
+  verify_body<true>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
+}
+__global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
+                                                     uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
+                                                     uint64_t mask, uint32_t* __restrict__ fail) {
+  verify_body<false>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
 }
 
 // Device-gated verify: one quad per segment of a unit, the launch's units (all of the arena's part shape) along the
@@ -944,11 +954,14 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
   return int(hipGetLastError());
 }
 
-// Whether a launch streams its segments: a check those of 1 and 2 KiB, the copy (which touches `bytes`, twice its units')
-// also others of whole chunk pairs, up to 4 KiB and 80 MB. Checks, streamed / chain loop, us in a loop on changing buffers:
-// 8.6 MB in 1.5 KiB segments 5.4 / 4.5, 8.4 MB in 4 KiB segments 7.9 / 6.4, 62 MB in 512-byte ones 11.9 / 10.9 (a wave's
-// pieces lie far apart, or a wave ends after one pair). The copy: 17 MB moved in 4 KiB segments 11.4 / 13.8, in 1.5 KiB
-// ones 7.7 / 8.0.
+// Whether a launch that touches `bytes` (the copy: twice its units') streams its segments: those of 2 KiB; where every part
+// lies on whole cache lines, checks above 80 MB those of 1 KiB too, the copy those of 512 bytes to 4 KiB in whole chunk pairs
+// (above 80 MB only 1 KiB). Streamed / chain loop, us in a loop on changing buffers:
+//  * Checks: 8.6 MB in 1.5 KiB segments 5.4 / 4.5, 8.4 MB in 4 KiB ones 7.9 / 6.4, 62 MB in 512-byte ones 11.9 / 10.9 (a
+//    wave's pieces lie far apart, or a wave ends after one pair); 1 KiB: 61 MB 11.5 / 10.9, 182 MB 29.6 / 31.7, but 148 MB
+//    that start in the middle of lines 31.0 / 27.0 (every chunk shares its ends' lines with its neighbours).
+//  * The copy: 17 MB moved in 4 KiB segments 11.4 / 13.8, in 1.5 KiB ones 7.7 / 8.0, 119 MB in 1 KiB ones 22.3 / 30.7; off
+//    the lines 53 MB in 4 KiB ones 20.5 / 16.7, in 1 KiB ones 14.7 / 13.2, in 2 KiB ones 14.1 / 14.6.
 //
 // One form for all sizes: two buffers a wave, reads past the caches, stores (the copy's) through them. Tried against it,
 // in workgroups of four waves, us (in a loop on changing buffers / one launch after other reads):
@@ -962,19 +975,20 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * Non-temporal stores, likewise: eight staged units (399 MB moved) 71.4 us against 78.5 in the loop, 75.2 against 65.1
 //    after other reads.
 constexpr uint64_t kNearBytes = 80000000;
-static bool check_streams(uint64_t seg_bytes) { return seg_bytes == 1024 || seg_bytes == 2048; }
-static bool copy_streams(uint64_t seg_bytes, uint64_t bytes) {
-  return check_streams(seg_bytes) || (seg_bytes % 512 == 0 && seg_bytes <= 4096 && bytes <= kNearBytes);
+static bool check_streams(uint64_t seg_bytes, uint64_t bytes) {
+  return seg_bytes == 2048 || (seg_bytes == 1024 && bytes > kNearBytes);
 }
-// Whether every part of every unit of the launch lies 16-byte aligned. One that does not streams wave by wave only above
-// 80 MB (102 MB, a third of it unaligned: 16.0 us against 18.9 for the chain loop on the same buffers); below, the chain
-// loop's kernel with its 8 waves on a SIMD is the better one (8.5 MB 5.2 us, wave by wave 5.8; 34 MB 7.7 / 7.9).
-static bool aligned16(const DgVerifyLaunch& a) {
+static bool copy_streams(uint64_t seg_bytes, uint64_t bytes) {
+  return bytes <= kNearBytes ? seg_bytes % 512 == 0 && seg_bytes <= 4096 : seg_bytes == 1024 || seg_bytes == 2048;
+}
+static uint32_t stream_align(uint64_t seg_bytes) { return seg_bytes == 2048 ? 16 : 128; }
+// Whether every part of every unit of the launch lies at a multiple of `align`.
+static bool aligned(const DgVerifyLaunch& a, uint32_t align) {
   for (uint32_t p = 0; p < a.n_parts; ++p) {
-    if (reinterpret_cast<uintptr_t>(a.arena[p]) % 16 != 0) return false;
-    if (a.part_bytes[p] % 16 == 0) continue;
+    if (reinterpret_cast<uintptr_t>(a.arena[p]) % align != 0) return false;
+    if (a.part_bytes[p] % align == 0) continue;
     for (uint32_t u = 0; u < a.n; ++u)
-      if (uint64_t(a.slots[u]) * a.part_bytes[p] % 16 != 0) return false;
+      if (uint64_t(a.slots[u]) * a.part_bytes[p] % align != 0) return false;
   }
   return true;
 }
@@ -1002,7 +1016,12 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  const bool stream_it = check_streams(a.seg_bytes) && (a.n * a.unit_bytes > kNearBytes || aligned16(a));
+  // An arena that is not aligned streams wave by wave only above 80 MB in 2 KiB segments (102 MB, a third of it unaligned:
+  // 16.0 us against 18.9 for the chain loop on the same buffers); else the chain loop's kernel with its 8 waves on a SIMD
+  // is the better one (8.5 MB 5.2 us, wave by wave 5.8; 34 MB 7.7 / 7.9).
+  const uint64_t bytes = a.n * a.unit_bytes;
+  const bool stream_it = check_streams(a.seg_bytes, bytes) &&
+                         (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
   auto* k = stream_it ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
   return e ? e : launch_publish(a, stream);
@@ -1015,7 +1034,13 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
   const uint32_t threads = 256;
   const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
-  auto* k = copy_streams(a.seg_bytes, 2 * a.n * a.unit_bytes) ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
+  bool stream_it = copy_streams(a.seg_bytes, 2 * a.n * a.unit_bytes);
+  if (stream_it && a.seg_bytes != 2048) {  // (2 KiB: its waves look for themselves)
+    const uint32_t align = stream_align(a.seg_bytes);
+    stream_it = aligned(a, align) && reinterpret_cast<uintptr_t>(src) % align == 0 && (a.n == 1 || a.unit_bytes % align == 0);
+    for (uint32_t p = 0; p + 1 < a.n_parts; ++p) stream_it = stream_it && a.part_bytes[p] % align == 0;
+  }
+  auto* k = stream_it ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
   const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
                              static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
@@ -1028,9 +1053,10 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = check_streams(seg_bytes) ? dev::verify_kernel<true> : dev::verify_kernel<false>;
+  auto* k = check_streams(seg_bytes, n_segments * seg_bytes) ? dev::verify_lds_kernel : dev::verify_kernel;
+  const uint64_t mask = stream_align(seg_bytes) - 1;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
-                      shift, fail_dev);
+                      shift, mask, fail_dev);
 }
 
 }  // namespace tsa
