@@ -17,16 +17,18 @@ namespace dev {
 // scalar loads: block by block, a chain of dependent reads ahead of every 16 KiB cost a tenth of a large launch.
 //
 // Reads go past the caches (each byte is read once), stores do not (the engine reads the slot next). The other ways were
-// faster only in an unbroken run of launches on changing buffers: cached reads 8.9 us against 10.7 for one unit of 24.8
-// MB, non-temporal stores 65.8 against 73.8 for eight. On its own, after a kernel has left the L2 full of written lines,
-// the first takes 17.0 us against 13.0 (the reads drive those lines out); after other reads the second takes 67.8 against
-// 62.0, and a 256 MiB copy 90.4 against 79.4.
+// faster only in an unbroken run of launches on changing buffers: cached reads 8.9 us against 10.3 for one unit of 24.8
+// MB, non-temporal stores 65.6 against 75.0 for eight. On its own, after a kernel has left the L2 full of written lines,
+// the first takes 16.9 us against 13.0 (the reads drive those lines out); after other reads the second takes 67.8 against
+// 62.5, and a 256 MiB copy 90.4 against 79.4.
 constexpr uint32_t kBlock = TSA_SCATTER_BLOCK_BYTES;
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kPerLane = kBlock / (16 * kThreads);  // 4
 
-__global__ __launch_bounds__(kThreads) void scatter_kernel(const TsaScatterJob* __restrict__ jobs, uint32_t n_jobs,
-                                                           uint64_t n_blocks) {
+// Held to 8 waves per SIMD: unbounded, the whole entry took the kernel from 54 to 72 registers and 7 waves, so that 2048
+// workgroups no longer ran at once (63 MB moved 14.8 us, with 54 registers 13.8, held 12.8).
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void scatter_kernel(
+    const TsaScatterJob* __restrict__ jobs, uint32_t n_jobs, uint64_t n_blocks) {
   const uint64_t blk = blockIdx.x;
   if (blk >= n_blocks) return;
   const uint32_t at = last_at_most(n_jobs, blk, [&](uint32_t i) { return jobs[i].block_first; });
