@@ -724,10 +724,9 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
   uint32_t ui = last_at_most(n_units, s0, [&](uint32_t i) { return units[i].seg_first; });
   HostSeg g;
   const uint64_t after = ui + 1 < n_units ? units[ui + 1].seg_first : ~0ull;
-  const TsaVerifyUnit un = units[ui];  // (whole and at once: with scalar loads, one memory latency)
-  if (after >= end) {
-    if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
-  } else {
+  TsaVerifyUnit un = units[ui];  // (whole and at once: with scalar loads, one memory latency)
+  const bool one = after >= end;  // the wave's segments are one unit's
+  if (!one) {
     // The quad's unit: the next 16 units' first segments in one read, counted up to the quad's own (unit by unit, 200
     // units of one segment each were 16 reads one behind the other: 8.6 us, 7.2 like this).
     const uint64_t base = ui + 1;
@@ -741,10 +740,15 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
         ui += seen <= s;
       }
     }
-    if (s < end) {
-      const TsaVerifyUnit mine = units[ui];
-      g = host_segment(mine, ui, s, seg_bytes, shift, fail, q);
-    }
+  }
+  if constexpr (kLds) {  // (one copy of the code for both: a first launch waits for it)
+    if (!one) un = units[ui];
+    if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
+  } else if (one) {  // (with the entry in scalar registers: 187 MB in 512-byte segments 31.7 us, 33.4 with it in vector ones)
+    if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
+  } else if (s < end) {
+    const TsaVerifyUnit mine = units[ui];
+    g = host_segment(mine, ui, s, seg_bytes, shift, fail, q);
   }
   if (__ballot(g.live) == 0) return;
   uint64_t v = 0, next = 0;
