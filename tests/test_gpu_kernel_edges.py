@@ -80,13 +80,13 @@ def test_synth_edges(gpu, kind, words, offset):
 # The checks by segment size and by size: two chunk buffers a wave (2 KiB segments; on whole cache lines 1 KiB ones above 80
 # MB and, in the copy, any whole pair of 256-byte chunks up to 4 KiB and 80 MB, above 1 KiB), the chain loop (other
 # segments; up to 80 MB also arenas with a part that is 8-byte aligned; above, and in batches and the copy, the waves
-# that hold one); parts that end inside a segment, inside a stripe, or are none.
+# that hold one); units in rows of workgroups or packed; parts that end inside a segment, inside a stripe, or are none.
 SHAPES = [
     (1, [2048], 2048), (1, [32], 2048), (2, [8], 2048), (1, [2080, 40], 2048), (5, [65568, 4096, 1000], 2048),
     (64, [30 * 2048 + 32, 96], 2048), (3, [2048 * 17, 2048 * 15 + 64, 32, 2048], 2048), (3, [(8 << 20) + 32, 1 << 20], 2048),
     (3, [28 << 20, (3 << 20) + 48], 2048), (3, [45 << 20, 4096 + 24], 2048), (2, [65536, 2048 + 1008], 512), (3, [65536 + 96, 1024 * 16], 1024),
     (2, [9 << 20, 1024 * 3 + 8], 1024), (3, [1536 * 40 + 32, 1536 * 16 - 8], 1536), (2, [1 << 20, 4096 * 3 + 56], 4096), (2, [1 << 20, 4096 * 3 + 128], 4096),
-    (1, [65536, 40], 4096), (2, [65536 + 64, 128], 1536),
+    (1, [65536, 40], 4096), (2, [65536 + 64, 128], 1536), (64, [530016, 40], 2048), (70, [530016, 48], 2048),
     (3, [28 << 20, 4096 + 16], 4096), (3, [28 << 20, (3 << 20) + 1000], 1024),
     (3, [44 << 20, (3 << 20) + 48], 1024), (2, [44 << 20, (3 << 20) + 128], 1024), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
 ]

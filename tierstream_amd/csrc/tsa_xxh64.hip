@@ -789,10 +789,11 @@ __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __rest
   verify_body<false>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
 }
 
-// Device-gated verify: one quad per segment of a unit, the launch's units (all of the arena's part shape) along the
-// grid's y, so that a wave has one unit: its key and slot are scalar, and no segment index is divided. kCopy (the staged
-// units' fused scatter): unit u's bytes are read from src + u x unit_bytes, where its parts lie back to back, and
-// written to their arena slot as they are hashed; the last segment's lane 0 also moves the unit's tail.
+// Device-gated verify: one quad per segment of a unit, the launch's units (all of the arena's part shape) along the grid's
+// y or packed, each from a wave of its own on, so that a wave has one unit: its key and slot are scalar, and no segment
+// index is divided. kCopy (the staged units' fused scatter): unit u's bytes are read from
+// src + u x unit_bytes, where its parts lie back to back, and written to their arena slot as they are hashed; the last
+// segment's lane 0 also moves the unit's tail.
 struct DgSeg {
   const uint64_t* state = nullptr;
   uint64_t digest = 0;
@@ -805,12 +806,29 @@ struct DgSeg {
   uint32_t tail_len = 0;
 };
 
+// The wave's unit and its first segment there. unit_waves: each unit's waves, one unit right behind the other (0: a row of the
+// grid each).
+struct DgWave {
+  uint32_t u = 0;
+  uint64_t first = 0;
+};
+__device__ __forceinline__ DgWave dg_wave(uint32_t unit_waves) {
+  DgWave w;
+  uint32_t k = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  w.u = blockIdx.y;
+  if (unit_waves) {
+    w.u = __builtin_amdgcn_readfirstlane(k / unit_waves);
+    k -= w.u * unit_waves;
+  }
+  w.first = uint64_t(k) * 16;
+  return w;
+}
+
 // (The part's fields are carried along the walk over the parts with constant indices, which keeps every read of the
 // launch's arguments a scalar load.)
 template <bool kCopy>
-__device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsigned char* src, uint64_t local) {
+__device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsigned char* src, uint32_t u, uint64_t local) {
   DgSeg g;
-  const uint32_t u = blockIdx.y;
   const uint64_t key = a.keys[u];
   const int32_t slot = a.slots[u];
   g.live = local < a.unit_segs;
@@ -851,8 +869,8 @@ __device__ __forceinline__ DgSeg dg_segment(const DgVerifyLaunch& a, const unsig
 
 // The segment's check (the next checkpoint, or for the unit's last segment the digest) and the gate.
 template <bool kCopy>
-__device__ __forceinline__ void dg_finish(const DgVerifyLaunch& a, const DgSeg& g, const Tail& tail, uint64_t v, uint64_t next,
-                                          uint32_t q) {
+__device__ __forceinline__ void dg_finish(const DgVerifyLaunch& a, uint32_t u, const DgSeg& g, const Tail& tail, uint64_t v,
+                                          uint64_t next, uint32_t q) {
   uint64_t all[4];
   const uint32_t base4 = threadIdx.x & ~3u;
 #pragma unroll
@@ -867,7 +885,7 @@ __device__ __forceinline__ void dg_finish(const DgVerifyLaunch& a, const DgSeg& 
     }
   }
   if (bad) {
-    atomicOr(a.fail + blockIdx.y, 1u);
+    atomicOr(a.fail + u, 1u);
     if (a.abort) {  // the gate: the token fails before the layer's ready word is written
       if (atomicCAS(a.err_code, 0u, a.err) == 0u) atomicExch(a.err_aux, a.aux);
       atomicExch(a.abort, 1u);
@@ -892,10 +910,11 @@ __global__ __launch_bounds__(64) void dg_publish_kernel(const DgVerifyLaunch a) 
 }
 
 template <bool kCopy>
-__device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, const unsigned char* src) {
-  const uint64_t gid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const uint32_t q = uint32_t(gid & 3u);
-  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
+__device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, uint32_t unit_waves, const unsigned char* src) {
+  const DgWave w = dg_wave(unit_waves);
+  if (w.u >= a.n || w.first >= a.unit_segs) return;  // (the whole wave)
+  const uint32_t q = threadIdx.x & 3u;
+  const DgSeg g = dg_segment<kCopy>(a, src, w.u, w.first + ((threadIdx.x & 63u) >> 2));
   uint64_t v = 0, next = 0;
   if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
@@ -903,20 +922,23 @@ __device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, const uns
   }
   Tail tail;
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
-  dg_finish<kCopy>(a, g, tail, v, next, q);
+  dg_finish<kCopy>(a, w.u, g, tail, v, next, q);
 }
-__global__ TSA_VERIFY_BOUNDS void dg_verify_kernel(const DgVerifyLaunch a) { dg_chain_body<false>(a, nullptr); }
-__global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_chain_body<true>(a, src);
+__global__ TSA_VERIFY_BOUNDS void dg_verify_kernel(const DgVerifyLaunch a, uint32_t unit_waves) {
+  dg_chain_body<false>(a, unit_waves, nullptr);
+}
+__global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch a, uint32_t unit_waves,
+                                                           const unsigned char* src) {
+  dg_chain_body<true>(a, unit_waves, src);
 }
 
 template <bool kCopy>
-__device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsigned char* src) {
+__device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, uint32_t unit_waves, const unsigned char* src) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
-  const uint64_t gid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
-  if ((gid & ~63ull) >> 2 >= a.unit_segs) return;  // (the whole wave)
-  const uint32_t q = uint32_t(gid & 3u);
-  const DgSeg g = dg_segment<kCopy>(a, src, gid >> 2);
+  const DgWave w = dg_wave(unit_waves);
+  if (w.u >= a.n || w.first >= a.unit_segs) return;  // (the whole wave)
+  const uint32_t q = threadIdx.x & 3u;
+  const DgSeg g = dg_segment<kCopy>(a, src, w.u, w.first + ((threadIdx.x & 63u) >> 2));
   Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
@@ -927,11 +949,14 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, const unsig
     next = g.last ? 0 : g.state[4 + q];
     v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
   }
-  dg_finish<kCopy>(a, g, tail, v, next, q);
+  dg_finish<kCopy>(a, w.u, g, tail, v, next, q);
 }
-__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a) { dg_lds_body<false>(a, nullptr); }
-__global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, const unsigned char* src) {
-  dg_lds_body<true>(a, src);
+__global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves) {
+  dg_lds_body<false>(a, unit_waves, nullptr);
+}
+__global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves,
+                                                                    const unsigned char* src) {
+  dg_lds_body<true>(a, unit_waves, src);
 }
 
 }  // namespace dev
@@ -997,6 +1022,19 @@ static bool aligned(const DgVerifyLaunch& a, uint32_t align) {
   return true;
 }
 
+// A row of whole workgroups for each unit while that is no more of them than the chip has CUs (64 units of one segment 5.8
+// us, packed 6.1), else the units' waves one right behind the other: 60 units of 51 waves in rows of 13 workgroups are 780,
+// so that some CUs get four, packed 765, three each (100 MB 23.1 us, packed 21.2).
+constexpr uint64_t kCus = 256;
+static bool dg_grid(const DgVerifyLaunch& a, dim3* grid, uint32_t* unit_waves) {
+  const uint64_t own = (a.unit_segs + 15) / 16, rows = (own + 3) / 4, packed = (a.n * own + 3) / 4;
+  if (a.n * rows > 0x3fffffffull) return false;
+  const bool pack = a.n > 1 && a.n * rows > kCus;
+  *unit_waves = pack ? uint32_t(own) : 0;
+  *grid = pack ? dim3(uint32_t(packed)) : dim3(uint32_t(rows), a.n);
+  return true;
+}
+
 static int launch_publish(const DgVerifyLaunch& a, hipStream_t stream) {
   if (!a.publish || (!a.slot_of && !a.ready)) return 0;
   hipLaunchKernelGGL(dev::dg_publish_kernel, dim3(1), dim3(64), 0, stream, a);
@@ -1017,9 +1055,9 @@ static int launch_timed(K* k, dim3 grid, uint32_t threads, hipStream_t stream, h
 int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4) return int(hipErrorInvalidValue);
-  const uint32_t threads = 256;
-  const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
-  if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
+  dim3 grid;
+  uint32_t waves = 0;
+  if (!dg_grid(a, &grid, &waves)) return int(hipErrorInvalidValue);
   // An arena that is not aligned streams wave by wave only above 80 MB in 2 KiB segments (102 MB, a third of it unaligned:
   // 16.0 us against 18.9 for the chain loop on the same buffers); else the chain loop's kernel with its 8 waves on a SIMD
   // is the better one (8.5 MB 5.2 us, wave by wave 5.8; 34 MB 7.7 / 7.9).
@@ -1027,7 +1065,7 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const bool stream_it = check_streams(a.seg_bytes, bytes) &&
                          (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
   auto* k = stream_it ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
-  const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a);
+  const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves);
   return e ? e : launch_publish(a, stream);
 }
 
@@ -1035,9 +1073,9 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
                              hipEvent_t stop) {
   if (a.n == 0 || a.unit_segs == 0) return 0;
   if (a.n > kDgVerifyMax || a.n_parts == 0 || a.n_parts > 4 || !src) return int(hipErrorInvalidValue);
-  const uint32_t threads = 256;
-  const uint64_t blocks = (a.unit_segs * 4 + threads - 1) / threads;
-  if (blocks > 0x7fffffffull / a.n) return int(hipErrorInvalidValue);
+  dim3 grid;
+  uint32_t waves = 0;
+  if (!dg_grid(a, &grid, &waves)) return int(hipErrorInvalidValue);
   bool stream_it = copy_streams(a.seg_bytes, 2 * a.n * a.unit_bytes);
   if (stream_it && a.seg_bytes != 2048) {  // (2 KiB: its waves look for themselves)
     const uint32_t align = stream_align(a.seg_bytes);
@@ -1045,8 +1083,7 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
     for (uint32_t p = 0; p + 1 < a.n_parts; ++p) stream_it = stream_it && a.part_bytes[p] % align == 0;
   }
   auto* k = stream_it ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
-  const int e = launch_timed(k, dim3(uint32_t(blocks), a.n), threads, stream, start, stop, a,
-                             static_cast<const unsigned char*>(src));
+  const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves, static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
 }
 
