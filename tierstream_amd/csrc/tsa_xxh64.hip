@@ -806,17 +806,18 @@ struct DgSeg {
   uint32_t tail_len = 0;
 };
 
-// The wave's unit and its first segment there. unit_waves: each unit's waves, one unit right behind the other (0: a row of the
-// grid each).
+// The wave's unit and its first segment there: kPack, each unit's unit_waves waves right behind the last one's; else a row of
+// the grid for each unit.
 struct DgWave {
   uint32_t u = 0;
   uint64_t first = 0;
 };
+template <bool kPack>
 __device__ __forceinline__ DgWave dg_wave(uint32_t unit_waves) {
   DgWave w;
   uint32_t k = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   w.u = blockIdx.y;
-  if (unit_waves) {
+  if (kPack) {
     w.u = __builtin_amdgcn_readfirstlane(k / unit_waves);
     k -= w.u * unit_waves;
   }
@@ -909,10 +910,10 @@ __global__ __launch_bounds__(64) void dg_publish_kernel(const DgVerifyLaunch a) 
   }
 }
 
-template <bool kCopy>
+template <bool kPack, bool kCopy>
 __device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, uint32_t unit_waves, const unsigned char* src) {
-  const DgWave w = dg_wave(unit_waves);
-  if (w.u >= a.n || w.first >= a.unit_segs) return;  // (the whole wave)
+  const DgWave w = dg_wave<kPack>(unit_waves);
+  if ((kPack && w.u >= a.n) || w.first >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = threadIdx.x & 3u;
   const DgSeg g = dg_segment<kCopy>(a, src, w.u, w.first + ((threadIdx.x & 63u) >> 2));
   uint64_t v = 0, next = 0;
@@ -924,19 +925,21 @@ __device__ __forceinline__ void dg_chain_body(const DgVerifyLaunch& a, uint32_t 
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   dg_finish<kCopy>(a, w.u, g, tail, v, next, q);
 }
+template <bool kPack>
 __global__ TSA_VERIFY_BOUNDS void dg_verify_kernel(const DgVerifyLaunch a, uint32_t unit_waves) {
-  dg_chain_body<false>(a, unit_waves, nullptr);
+  dg_chain_body<kPack, false>(a, unit_waves, nullptr);
 }
+template <bool kPack>
 __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch a, uint32_t unit_waves,
                                                            const unsigned char* src) {
-  dg_chain_body<true>(a, unit_waves, src);
+  dg_chain_body<kPack, true>(a, unit_waves, src);
 }
 
-template <bool kCopy>
+template <bool kPack, bool kCopy>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, uint32_t unit_waves, const unsigned char* src) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
-  const DgWave w = dg_wave(unit_waves);
-  if (w.u >= a.n || w.first >= a.unit_segs) return;  // (the whole wave)
+  const DgWave w = dg_wave<kPack>(unit_waves);
+  if ((kPack && w.u >= a.n) || w.first >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = threadIdx.x & 3u;
   const DgSeg g = dg_segment<kCopy>(a, src, w.u, w.first + ((threadIdx.x & 63u) >> 2));
   Tail tail;  // (read ahead of the chains: at the end it would be one more memory latency)
@@ -951,12 +954,14 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, uint32_t un
   }
   dg_finish<kCopy>(a, w.u, g, tail, v, next, q);
 }
+template <bool kPack>
 __global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves) {
-  dg_lds_body<false>(a, unit_waves, nullptr);
+  dg_lds_body<kPack, false>(a, unit_waves, nullptr);
 }
+template <bool kPack>
 __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves,
                                                                     const unsigned char* src) {
-  dg_lds_body<true>(a, unit_waves, src);
+  dg_lds_body<kPack, true>(a, unit_waves, src);
 }
 
 }  // namespace dev
@@ -1064,7 +1069,8 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint64_t bytes = a.n * a.unit_bytes;
   const bool stream_it = check_streams(a.seg_bytes, bytes) &&
                          (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
-  auto* k = stream_it ? dev::dg_verify_lds_kernel : dev::dg_verify_kernel;
+  auto* k = stream_it ? (waves ? dev::dg_verify_lds_kernel<true> : dev::dg_verify_lds_kernel<false>)
+                      : (waves ? dev::dg_verify_kernel<true> : dev::dg_verify_kernel<false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves);
   return e ? e : launch_publish(a, stream);
 }
@@ -1082,7 +1088,8 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
     stream_it = aligned(a, align) && reinterpret_cast<uintptr_t>(src) % align == 0 && (a.n == 1 || a.unit_bytes % align == 0);
     for (uint32_t p = 0; p + 1 < a.n_parts; ++p) stream_it = stream_it && a.part_bytes[p] % align == 0;
   }
-  auto* k = stream_it ? dev::dg_scatter_verify_lds_kernel : dev::dg_scatter_verify_kernel;
+  auto* k = stream_it ? (waves ? dev::dg_scatter_verify_lds_kernel<true> : dev::dg_scatter_verify_lds_kernel<false>)
+                      : (waves ? dev::dg_scatter_verify_kernel<true> : dev::dg_scatter_verify_kernel<false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves, static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
 }
