@@ -120,11 +120,9 @@ __device__ __forceinline__ uint64_t xfinal(const uint64_t v[4], uint64_t total, 
 // They are ordinary cached loads: the quad reads 32 bytes of a 128-byte line per stripe and the next three stripes
 // read the rest of it, so the line must stay in the CU's cache (a streaming hint that skips it cost 40 % on gfx950).
 //
-// Measured on one 336 MiB unit (8 KiB segments): this loop reads at 5.8 TB/s, 95 % of what a fully coalesced 16-byte
-// streaming read of the same bytes reaches in one launch (6.1 TB/s); the rounds alone (no loads) run at 17 TB/s. So
-// the kernel is bound by the read, not the multiplies, and neither a software-pipelined nor an LDS-staged variant
-// (coalesced 16-byte loads into LDS, chains run from LDS) beat it. Sixteen stripes a block: with 8, 25 MB of
-// 8-byte aligned units took 8.3 us against 7.6; with 32, 34 MB of ragged ones 12.0 against 10.7.
+// Measured on one 336 MiB unit (8 KiB segments): this loop reads at 5.8 TB/s; the rounds alone (no loads) run at 17 TB/s, so
+// it is bound by the read, not the multiplies. The streamed check below reads aligned segments at 6.4 TB/s. Sixteen stripes a
+// block: with 8, 25 MB of 8-byte aligned units took 8.3 us against 7.6; with 32, 34 MB of ragged ones 12.0 against 10.7.
 constexpr int kBlock = 16;
 
 // kCopy: each word read is also stored at the same offset from d (the staged unit's bytes into their arena slot while
@@ -449,7 +447,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
   if (ends) out[u] = xfinal(all, us.bytes, tail);
 }
 
-// ---- The LDS-streamed check (segments of a multiple of 512 bytes) ----
+// ---- The LDS-streamed check ----
 //
 // The chain loop above reads 8 bytes per lane at a 32-byte stride: every load instruction of a wave touches 16 lines
 // (one per quad) and relies on the CU cache to keep each line for the next three. Here every wave streams its 16
@@ -466,15 +464,16 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
 // The loads are inline assembly, so the compiler neither waits for them nor knows them; each chunk waits for its own
 // loads with an explicit vmcnt (loads complete in order, and a load or store of the compiler's among them only makes
 // the wait longer). Lanes whose piece lies past their segment's stripes load an earlier piece again (never out of
-// bounds), and every wave issues the same number of loads, which the vmcnt counts rely on. The instruction's offset
-// moves both addresses, so the chunks of a wave of whole segments take no address arithmetic. A chunk that every
-// segment has whole or not at all is hashed without a select per round: waves at the end of a part are as fast as the
-// others (with both costs in them they were the launch's last: 8 MB in 5.5 us instead of 6.3).
+// bounds), and every wave issues the same number of loads, which the vmcnt counts rely on. A chunk that every segment has
+// whole or not at all is hashed without a select per round: waves at the end of a part are as fast as the others (with
+// both costs in them they were the launch's last: 8 MB in 5.5 us instead of 6.3).
 //
-// What bounds it: reading, from about 50 MB on (336 MiB 55.8 us, 6.4 TB/s); below, one launch and one to four memory
-// latencies (192 KiB 4.9 us, of which a launch of nothing takes 3.7).
-constexpr uint32_t kChunkBuffers = 2 * 4096;              // per wave
-constexpr uint32_t kWaveLds = kChunkBuffers + 64 * 16;  // and 64 bytes of checkpoints per quad behind them
+// What bounds it: reading, from about 50 MB on (336 MiB in 56.1 us on changing buffers, 6.4 TB/s); below, one launch and
+// four or five memory latencies (192 KiB 5.4 us, of which a launch of nothing takes 3.7).
+template <uint32_t kD>  // per wave: kD chunk buffers, and 64 bytes of checkpoints per quad behind them
+constexpr uint32_t wave_lds_bytes() {
+  return kD * 4096 + 64 * 16;
+}
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) u32x4 gu32x4_t;
@@ -522,16 +521,27 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Chunk by chunk, each when it has landed (the later ones' loads may still be in flight).
+template <uint32_t kD, uint32_t kC = 0, class F>
+__device__ __forceinline__ void drain(F&& hash) {
+  if constexpr (kC < kD) {
+    wait_loads<4 * (kD - 1 - kC)>();
+    hash(kC);
+    drain<kD, kC + 1>(hash);
+  }
+}
+
 // One wave's 16 segments (quad j's lanes 4 j + q hold segment j): where it is read and (kCopy) written, its stripes (0
 // hashes nothing and reads 16 bytes), its checkpoint (32 bytes, 64 when it is not the unit's last). Out: the
 // accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
-// go along with the first live segment and their results mean nothing. lds: the wave's kWaveLds.
+// go along with the first live segment and their results mean nothing. lds: the wave's wave_lds_bytes<kD>().
 //
-// Two chunk buffers go round: chunk c + 2 is loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0).
+// kD chunk buffers go round: chunk c + kD is loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0).
+template <uint32_t kD>
 __device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
-  return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWaveLds;
+  return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * wave_lds_bytes<kD>();
 }
-template <bool kCopy>
+template <uint32_t kD, bool kCopy>
 __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* from, unsigned char* to,
                                               uint32_t stripes, const uint64_t* state, bool last,
                                               unsigned char* lds, uint64_t* next) {
@@ -549,9 +559,9 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
   uint32_t most = stripes;  // as many rounds of the buffers as the wave's longest segment has
 #pragma unroll
   for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
-  const uint32_t chunks = max(2u, __builtin_amdgcn_readfirstlane((most + 15) / 16 * 2));
+  const uint32_t chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
   const bool whole = __all(!live || stripes == 8 * chunks);
-  lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kChunkBuffers);
+  lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
   // The lane's piece of load k (of segment 4k + i: quad 4k + i's lane 0 holds its source) in chunk 0, and how far its
   // segment has later ones: past that the lane loads the last one again, or (no stripe of its own) the segment's first.
   const unsigned char* src[4];
@@ -624,29 +634,27 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
       }
     }
   };
-  issue(0, 0);
-  issue(1, 1);
-  wait_loads<8>();
-  const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kChunkBuffers + j * 64);
+#pragma unroll
+  for (uint32_t c = 0; c < kD; ++c) issue(c, c);
+  wait_loads<4 * kD>();
+  const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kD * 4096 + j * 64);
   b = st[q] * P1inv;
   *next = st[4 + q];
-  for (uint32_t c = 0; c + 2 < chunks; c += 2) {
+  for (uint32_t c = 0; c + kD < chunks; c += kD) {
 #pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-      wait_loads<4>();
+    for (uint32_t i = 0; i < kD; ++i) {
+      wait_loads<4 * (kD - 1)>();
       if (kCopy) store(c + i, i);
       hash(c + i, i);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue(c + i + 2, i);
+      issue(c + i + kD, i);
     }
   }
-  const uint32_t c = chunks - 2;
-  wait_loads<4>();
-  if (kCopy) store(c, 0);
-  hash(c, 0);
-  wait_loads<0>();
-  if (kCopy) store(c + 1, 1);
-  hash(c + 1, 1);
+  const uint32_t c = chunks - kD;
+  drain<kD>([&](uint32_t i) {
+    if (kCopy) store(c + i, i);
+    hash(c + i, i);
+  });
   return b * P1;
 }
 
@@ -755,11 +763,11 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
   bool streamed = false;
   if constexpr (kLds) {
     streamed = __all(!g.live || (reinterpret_cast<uintptr_t>(g.from) & mask) == 0);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * wave_lds_bytes<2>()];
     if (streamed)
-      v = lds_check<false>(
+      v = lds_check<2, false>(
           g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
-          g.last, wave_lds(lds), &next);
+          g.last, wave_lds<2>(lds), &next);
   }
   if (!streamed && g.live) {
     // (global loads: with a generic one under way the compiler waits for all of a block's words before its first round)
@@ -935,9 +943,9 @@ __global__ TSA_VERIFY_BOUNDS void dg_scatter_verify_kernel(const DgVerifyLaunch 
   dg_chain_body<kPack, true>(a, unit_waves, src);
 }
 
-template <bool kPack, bool kCopy>
+template <uint32_t kD, bool kPack, bool kCopy>
 __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, uint32_t unit_waves, const unsigned char* src) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWaveLds];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * wave_lds_bytes<kD>()];
   const DgWave w = dg_wave<kPack>(unit_waves);
   if ((kPack && w.u >= a.n) || w.first >= a.unit_segs) return;  // (the whole wave)
   const uint32_t q = threadIdx.x & 3u;
@@ -946,22 +954,22 @@ __device__ __forceinline__ void dg_lds_body(const DgVerifyLaunch& a, uint32_t un
   if (g.last && q == 0) tail = load_tail(g.tail, g.tail_len);
   uint64_t v = 0, next = 0;
   if (__all(!g.live || (reinterpret_cast<uintptr_t>(g.from) | (kCopy ? reinterpret_cast<uintptr_t>(g.to) : 0)) % 16 == 0)) {
-    v = lds_check<kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
-                                  g.state, g.last, wave_lds(lds), &next);
+    v = lds_check<kD, kCopy>(g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), g.to, g.stripes,
+                                  g.state, g.last, wave_lds<kD>(lds), &next);
   } else if (g.live) {
     next = g.last ? 0 : g.state[4 + q];
     v = chain_t<kCopy>(g.state[q], g.from, g.to, g.stripes, q);
   }
   dg_finish<kCopy>(a, w.u, g, tail, v, next, q);
 }
-template <bool kPack>
+template <uint32_t kD, bool kPack>
 __global__ __launch_bounds__(256) void dg_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves) {
-  dg_lds_body<kPack, false>(a, unit_waves, nullptr);
+  dg_lds_body<kD, kPack, false>(a, unit_waves, nullptr);
 }
-template <bool kPack>
+template <uint32_t kD, bool kPack>
 __global__ __launch_bounds__(256) void dg_scatter_verify_lds_kernel(const DgVerifyLaunch a, uint32_t unit_waves,
                                                                     const unsigned char* src) {
-  dg_lds_body<kPack, true>(a, unit_waves, src);
+  dg_lds_body<kD, kPack, true>(a, unit_waves, src);
 }
 
 }  // namespace dev
@@ -997,12 +1005,15 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * The copy: 17 MB moved in 4 KiB segments 11.4 / 13.8, in 1.5 KiB ones 7.7 / 8.0, 119 MB in 1 KiB ones 22.3 / 30.7; off
 //    the lines 53 MB in 4 KiB ones 20.5 / 16.7, in 1 KiB ones 14.7 / 13.2, in 2 KiB ones 14.1 / 14.6.
 //
-// One form for all sizes: two buffers a wave, reads past the caches, stores (the copy's) through them. Tried against it,
-// in workgroups of four waves, us (in a loop on changing buffers / one launch after other reads):
-//  * Four buffers (70 KB of LDS a workgroup, two on a CU): 85 MB 16.0 / 19.9, two 15.5 / 19.0; 300 MB batch 48.4 / 53.0,
-//    two 47.8 / 50.6; with 1 KiB segments 54.5 / 59.0, two 50.0 / 52.1.
-//  * All of a segment's chunks in flight at once (132 KiB a workgroup): 64 waves 5.53 / 9.16, ring 5.44 / 9.04; 512 waves
-//    6.68 / 9.56, ring 6.58 / 9.44. Better only for a single wave (5.0 / 8.3, ring 5.1 / 9.2).
+// Two buffers a wave; four for the copy above 80 MB and for checks above it whose parts lie off the cache lines. Reads go past
+// the caches, stores (the copy's) through them. Measured in workgroups of four waves, us (in a loop on changing buffers / one
+// launch after other reads):
+//  * Four buffers, 70 KB of LDS a workgroup, two on a CU. On whole lines: 85 MB 16.0 / 19.9, two 15.5 / 19.0; 358 MB 56.9 /
+//    58.8, two 56.4 / 59.5; 307 MB batch 48.8 / 53.4, two 47.9 / 51.0. Off them: 358 MB 62.6 / 65.0, two 71.4 / 73.9; 178 MB
+//    32.1 / 37.7, two 35.0 / 41.8 (a batch's extents are not known here: two). The copy: 150 MB moved 28.8 / 31.6, two 30.0 /
+//    32.4; 50 MB moved 11.8 / 15.0, two 12.0 / 15.0.
+//  * All of a segment's chunks in flight at once (132 KiB a workgroup): 3 MB 6.26 / 12.6, two buffers 5.96 / 10.6; 12.8 MB
+//    6.98 / 12.4, two 6.40 / 10.5.
 //  * Cached reads, faster only in the loop (staged 24.8 MB unit 10.2 us against 12.0, 51 MB unit 9.8 / 10.4): after a
 //    kernel has left the L2 full of written lines, which they drive out, 19.7 us against 15.4 and 23.8 against 13.4; in
 //    decode tokens 14.5 against 14.9 and (48 MiB) 13.7 against 13.1.
@@ -1069,8 +1080,10 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint64_t bytes = a.n * a.unit_bytes;
   const bool stream_it = check_streams(a.seg_bytes, bytes) &&
                          (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
-  auto* k = stream_it ? (waves ? dev::dg_verify_lds_kernel<true> : dev::dg_verify_lds_kernel<false>)
-                      : (waves ? dev::dg_verify_kernel<true> : dev::dg_verify_kernel<false>);
+  const bool four = stream_it && bytes > kNearBytes && !aligned(a, 128);
+  auto* k = !stream_it ? (waves ? dev::dg_verify_kernel<true> : dev::dg_verify_kernel<false>)
+            : four     ? (waves ? dev::dg_verify_lds_kernel<4, true> : dev::dg_verify_lds_kernel<4, false>)
+                       : (waves ? dev::dg_verify_lds_kernel<2, true> : dev::dg_verify_lds_kernel<2, false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves);
   return e ? e : launch_publish(a, stream);
 }
@@ -1082,14 +1095,17 @@ int launch_dg_scatter_verify(const DgVerifyLaunch& a, const void* src, hipStream
   dim3 grid;
   uint32_t waves = 0;
   if (!dg_grid(a, &grid, &waves)) return int(hipErrorInvalidValue);
-  bool stream_it = copy_streams(a.seg_bytes, 2 * a.n * a.unit_bytes);
+  const uint64_t bytes = 2 * a.n * a.unit_bytes;
+  bool stream_it = copy_streams(a.seg_bytes, bytes);
   if (stream_it && a.seg_bytes != 2048) {  // (2 KiB: its waves look for themselves)
     const uint32_t align = stream_align(a.seg_bytes);
     stream_it = aligned(a, align) && reinterpret_cast<uintptr_t>(src) % align == 0 && (a.n == 1 || a.unit_bytes % align == 0);
     for (uint32_t p = 0; p + 1 < a.n_parts; ++p) stream_it = stream_it && a.part_bytes[p] % align == 0;
   }
-  auto* k = stream_it ? (waves ? dev::dg_scatter_verify_lds_kernel<true> : dev::dg_scatter_verify_lds_kernel<false>)
-                      : (waves ? dev::dg_scatter_verify_kernel<true> : dev::dg_scatter_verify_kernel<false>);
+  const bool four = bytes > kNearBytes;
+  auto* k = !stream_it ? (waves ? dev::dg_scatter_verify_kernel<true> : dev::dg_scatter_verify_kernel<false>)
+            : four     ? (waves ? dev::dg_scatter_verify_lds_kernel<4, true> : dev::dg_scatter_verify_lds_kernel<4, false>)
+                       : (waves ? dev::dg_scatter_verify_lds_kernel<2, true> : dev::dg_scatter_verify_lds_kernel<2, false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves, static_cast<const unsigned char*>(src));
   return e ? e : launch_publish(a, stream);
 }
