@@ -492,28 +492,37 @@ __device__ __forceinline__ void lds_load16(const unsigned char* g, uint32_t lds_
       : "v"(g), "s"(lds_addr)
       : "memory");
 }
-// A chunk: piece k of the lane at g[k] to lds_addr + 1024 k.
+// A chunk: piece k of the lane at g[k] + kAt to lds_addr + 1024 k (the instruction's offset moves both addresses).
+template <uint32_t kAt = 0>
 __device__ __forceinline__ void lds_load_chunk(const unsigned char* const g[4], uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %5\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off nt\n\t"
+      "global_load_lds_dwordx4 %1, off offset:%6 nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %2, off nt\n\t"
+      "global_load_lds_dwordx4 %2, off offset:%6 nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %3, off nt\n\t"
+      "global_load_lds_dwordx4 %3, off offset:%6 nt\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %4, off nt\n\t"
+      "global_load_lds_dwordx4 %4, off offset:%6 nt\n\t"
       "s_mov_b32 m0, %0\n\t"
       "s_nop 0"
       : "=&s"(save)
-      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr)
+      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "s"(lds_addr - kAt), "n"(kAt)
       : "memory", "scc");
+}
+
+template <uint32_t kD, uint32_t kC = 0>
+__device__ __forceinline__ void issue_all(const unsigned char* const g[4], uint32_t lds_off) {
+  if constexpr (kC < kD) {
+    lds_load_chunk<kC * 256>(g, lds_off + kC * 4096);
+    issue_all<kD, kC + 1>(g, lds_off);
+  }
 }
 
 template <int N>
@@ -536,7 +545,9 @@ __device__ __forceinline__ void drain(F&& hash) {
 // accumulator after the segment, and the next checkpoint's. All 64 lanes call it, at least one of them live; the others
 // go along with the first live segment and their results mean nothing. lds: the wave's wave_lds_bytes<kD>().
 //
-// kD chunk buffers go round: chunk c + kD is loaded when chunk c has been hashed (its LDS reads complete: lgkmcnt 0).
+// kD 2 or 4: as many chunk buffers go round, chunk c + kD loaded when chunk c has been hashed (its LDS reads complete:
+// lgkmcnt 0). kD 8: segments of up to 2 KiB, all their chunks in flight at once (not for the copy, whose stores the waits
+// would wait for).
 template <uint32_t kD>
 __device__ __forceinline__ unsigned char* wave_lds(unsigned char* lds) {  // the wave's part of its workgroup's
   return lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * wave_lds_bytes<kD>();
@@ -556,10 +567,15 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
   from = reinterpret_cast<const unsigned char*>(from_first(reinterpret_cast<uintptr_t>(from), reinterpret_cast<uintptr_t>(from)));
   state = reinterpret_cast<const uint64_t*>(from_first(reinterpret_cast<uintptr_t>(state), reinterpret_cast<uintptr_t>(state)));
   last = last || !live;
-  uint32_t most = stripes;  // as many rounds of the buffers as the wave's longest segment has
+  constexpr bool kAll = kD == 8;
+  static_assert(!kAll || !kCopy, "");
+  uint32_t chunks = kD;
+  if (!kAll) {  // as many rounds of the buffers as the wave's longest segment has
+    uint32_t most = stripes;
 #pragma unroll
-  for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
-  const uint32_t chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
+    for (uint32_t d = 4; d < 64; d *= 2) most = max(most, uint32_t(__shfl_xor(int(most), int(d), 64)));
+    chunks = max(kD, __builtin_amdgcn_readfirstlane((most + 8 * kD - 1) / (8 * kD) * kD));
+  }
   const bool whole = __all(!live || stripes == 8 * chunks);
   lds_load16(reinterpret_cast<const unsigned char*>(state) + (last ? q & 1u : q) * 16, lds_off + kD * 4096);
   // The lane's piece of load k (of segment 4k + i: quad 4k + i's lane 0 holds its source) in chunk 0, and how far its
@@ -634,13 +650,17 @@ __device__ __forceinline__ uint64_t lds_check(bool live, const unsigned char* fr
       }
     }
   };
-#pragma unroll
-  for (uint32_t c = 0; c < kD; ++c) issue(c, c);
+  if (kAll && whole) {
+    issue_all<kD>(src, lds_off);
+  } else {
+#pragma unroll (kAll ? 1 : kD)
+    for (uint32_t c = 0; c < kD; ++c) issue(c, c);
+  }
   wait_loads<4 * kD>();
   const uint64_t* st = reinterpret_cast<const uint64_t*>(lds + kD * 4096 + j * 64);
   b = st[q] * P1inv;
   *next = st[4 + q];
-  for (uint32_t c = 0; c + kD < chunks; c += kD) {
+  for (uint32_t c = 0; !kAll && c + kD < chunks; c += kD) {
 #pragma unroll
     for (uint32_t i = 0; i < kD; ++i) {
       wait_loads<4 * (kD - 1)>();
@@ -718,9 +738,10 @@ __device__ __forceinline__ HostSeg host_segment(const TsaVerifyUnit& un, uint32_
   g.total = un.total;
   return g;
 }
-// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kLds: waves
-// whose segments all start at a multiple of `mask` + 1 stream through LDS; any other runs the chain loop from memory.
-template <bool kLds>
+// One (unit, segment) per quad. seg_first is the prefix sum of segments over the launch's units (ascending). kD: as for
+// lds_check, in waves whose segments all start at a multiple of `mask` + 1; any other wave, and every one with kD 0, runs the
+// chain loop from memory.
+template <uint32_t kD>
 __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ units, uint32_t n_units, uint64_t n_segments,
                                             uint64_t seg_bytes, uint32_t shift, uint64_t mask,
                                             uint32_t* __restrict__ fail) {
@@ -749,7 +770,7 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
       }
     }
   }
-  if constexpr (kLds) {  // (one copy of the code for both: a first launch waits for it)
+  if constexpr (kD != 0) {  // (one copy of the code for both: a first launch waits for it)
     if (!one) un = units[ui];
     if (s < end) g = host_segment(un, ui, s, seg_bytes, shift, fail, q);
   } else if (one) {  // (with the entry in scalar registers: 187 MB in 512-byte segments 31.7 us, 33.4 with it in vector ones)
@@ -761,13 +782,13 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
   if (__ballot(g.live) == 0) return;
   uint64_t v = 0, next = 0;
   bool streamed = false;
-  if constexpr (kLds) {
+  if constexpr (kD != 0) {
     streamed = __all(!g.live || (reinterpret_cast<uintptr_t>(g.from) & mask) == 0);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * wave_lds_bytes<2>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * wave_lds_bytes<kD>()];
     if (streamed)
-      v = lds_check<2, false>(
+      v = lds_check<kD, false>(
           g.live, g.stripes ? g.from : reinterpret_cast<const unsigned char*>(g.state), nullptr, uint32_t(g.stripes), g.state,
-          g.last, wave_lds<2>(lds), &next);
+          g.last, wave_lds<kD>(lds), &next);
   }
   if (!streamed && g.live) {
     // (global loads: with a generic one under way the compiler waits for all of a block's words before its first round)
@@ -786,15 +807,16 @@ __device__ __forceinline__ void verify_body(const TsaVerifyUnit* __restrict__ un
     if (xfinal(all, g.total, g.tail) != g.digest) atomicOr(fail + g.ui, 1u);
   }
 }
+template <uint32_t kD>
 __global__ __launch_bounds__(256) void verify_lds_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
                                                          uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
                                                          uint64_t mask, uint32_t* __restrict__ fail) {
-  verify_body<true>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
+  verify_body<kD>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
 }
 __global__ __launch_bounds__(256) void verify_kernel(const TsaVerifyUnit* __restrict__ units, uint32_t n_units,
                                                      uint64_t n_segments, uint64_t seg_bytes, uint32_t shift,
                                                      uint64_t mask, uint32_t* __restrict__ fail) {
-  verify_body<false>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
+  verify_body<0>(units, n_units, n_segments, seg_bytes, shift, mask, fail);
 }
 
 // Device-gated verify: one quad per segment of a unit, the launch's units (all of the arena's part shape) along the grid's
@@ -1005,21 +1027,24 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //  * The copy: 17 MB moved in 4 KiB segments 11.4 / 13.8, in 1.5 KiB ones 7.7 / 8.0, 119 MB in 1 KiB ones 22.3 / 30.7; off
 //    the lines 53 MB in 4 KiB ones 20.5 / 16.7, in 1 KiB ones 14.7 / 13.2, in 2 KiB ones 14.1 / 14.6.
 //
-// Two buffers a wave; four for the copy above 80 MB and for checks above it whose parts lie off the cache lines. Reads go past
-// the caches, stores (the copy's) through them. Measured in workgroups of four waves, us (in a loop on changing buffers / one
+// Two buffers a wave; four for the copy above 80 MB and for checks above it whose parts lie off the cache lines; all of a
+// segment's chunks in flight for checks of units (batches) of up to 96 segments of 2 KiB. Reads go past the caches, stores (the copy's) through them. Measured in workgroups of four waves, us (in a loop on changing buffers / one
 // launch after other reads):
 //  * Four buffers, 70 KB of LDS a workgroup, two on a CU. On whole lines: 85 MB 16.0 / 19.9, two 15.5 / 19.0; 358 MB 56.9 /
 //    58.8, two 56.4 / 59.5; 307 MB batch 48.8 / 53.4, two 47.9 / 51.0. Off them: 358 MB 62.6 / 65.0, two 71.4 / 73.9; 178 MB
 //    32.1 / 37.7, two 35.0 / 41.8 (a batch's extents are not known here: two). The copy: 150 MB moved 28.8 / 31.6, two 30.0 /
 //    32.4; 50 MB moved 11.8 / 15.0, two 12.0 / 15.0.
-//  * All of a segment's chunks in flight at once (132 KiB a workgroup): 3 MB 6.26 / 12.6, two buffers 5.96 / 10.6; 12.8 MB
-//    6.98 / 12.4, two 6.40 / 10.5.
+//  * All chunks in flight, 132 KiB of LDS a workgroup: one unit of 32 KiB 4.77 / 8.1, two buffers 5.17 / 10.0; 192 KiB 5.18 /
+//    10.2, two 5.38 / 9.7; eight of them 5.51 / 9.3, two 5.79 / 9.5; a batch of 157 KB 5.44 / 10.9, two 5.71 / 11.4. But one
+//    unit of 256 KiB 5.45 / 10.3, two 5.38 / 9.6; 3 MB 6.26 / 12.6, two 5.96 / 10.6: a CU then waits for its four waves'
+//    chunks at once.
 //  * Cached reads, faster only in the loop (staged 24.8 MB unit 10.2 us against 12.0, 51 MB unit 9.8 / 10.4): after a
 //    kernel has left the L2 full of written lines, which they drive out, 19.7 us against 15.4 and 23.8 against 13.4; in
 //    decode tokens 14.5 against 14.9 and (48 MiB) 13.7 against 13.1.
 //  * Non-temporal stores, likewise: eight staged units (399 MB moved) 71.4 us against 78.5 in the loop, 75.2 against 65.1
 //    after other reads.
 constexpr uint64_t kNearBytes = 80000000;
+constexpr uint64_t kFewSegs = 96;
 static bool check_streams(uint64_t seg_bytes, uint64_t bytes) {
   return seg_bytes == 2048 || (seg_bytes == 1024 && bytes > kNearBytes);
 }
@@ -1080,8 +1105,10 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const uint64_t bytes = a.n * a.unit_bytes;
   const bool stream_it = check_streams(a.seg_bytes, bytes) &&
                          (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
+  const bool few = a.seg_bytes == 2048 && a.unit_segs <= kFewSegs;
   const bool four = stream_it && bytes > kNearBytes && !aligned(a, 128);
   auto* k = !stream_it ? (waves ? dev::dg_verify_kernel<true> : dev::dg_verify_kernel<false>)
+            : few      ? (waves ? dev::dg_verify_lds_kernel<8, true> : dev::dg_verify_lds_kernel<8, false>)
             : four     ? (waves ? dev::dg_verify_lds_kernel<4, true> : dev::dg_verify_lds_kernel<4, false>)
                        : (waves ? dev::dg_verify_lds_kernel<2, true> : dev::dg_verify_lds_kernel<2, false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves);
@@ -1117,7 +1144,9 @@ int launch_verify(const TsaVerifyUnit* units_dev, uint32_t n_units, uint64_t n_s
   const uint64_t blocks = (n_segments * 4 + threads - 1) / threads;
   if (blocks > 0x7fffffffull) return int(hipErrorInvalidValue);
   const uint32_t shift = seg_bytes & (seg_bytes - 1) ? 64 : uint32_t(__builtin_ctzll(seg_bytes));
-  auto* k = check_streams(seg_bytes, n_segments * seg_bytes) ? dev::verify_lds_kernel : dev::verify_kernel;
+  auto* k = !check_streams(seg_bytes, n_segments * seg_bytes) ? dev::verify_kernel
+            : seg_bytes == 2048 && n_segments <= kFewSegs     ? dev::verify_lds_kernel<8>
+                                                              : dev::verify_lds_kernel<2>;
   const uint64_t mask = stream_align(seg_bytes) - 1;
   return launch_timed(k, dim3(uint32_t(blocks)), threads, stream, start, stop, units_dev, n_units, n_segments, seg_bytes,
                       shift, mask, fail_dev);
