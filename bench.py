@@ -58,7 +58,7 @@ SCATTER_VERIFY_TRAFFIC_PER_UNIT = {24772608: 50273920}
 TRAFFIC_SOURCE = {("verify", 352321536): "profiles/dg_verify_lds_kernel_mixtral_unit_pmc.md",
                   ("verify", 24772608): "profiles/dg_scatter_verify_lds_kernel_deepseek_unit_pmc.md",
                   ("fused", 24772608): "profiles/dg_scatter_verify_lds_kernel_deepseek_unit_pmc.md"}
-# The host contract's verify_kernel: HBM bytes fetched per algorithmic byte hashed, keyed by unit bytes, from
+# The host contract's check (verify_lds_kernel; measured while it was one with verify_kernel): HBM bytes fetched per algorithmic byte hashed, keyed by unit bytes, from
 # rocprofv3 --pmc FETCH_SIZE over the bench's own timed steps (scaled as above): a full batch of 32 units fetches
 # 149,987.63 KiB x 2.0 = 307,174,656 B for 301,989,888 B of units (2 KiB checkpoint segments), nothing written
 # (profiles/verify_kernel_qwen3_host_pmc.md).
@@ -70,10 +70,15 @@ HOST_TRAFFIC_SOURCE = {9437184: "profiles/verify_kernel_qwen3_host_pmc.md",
 
 
 def dg_check_kernel(parts, seg, fused):
-    """The kernel the library launches for a device-gated check of this arena shape: the LDS-streamed one for 2 KiB
-    segments and 16-byte aligned parts of at least 16 bytes (the arena's parts are separate allocations), the chain
-    loop otherwise."""
-    lds = seg == 2048 and all(pb % 16 == 0 and pb >= 16 for pb in parts)
+    """The kernel the library launches for one unit's device-gated check in this arena shape (the arena's parts are
+    separate allocations): the LDS-streamed one for 2 KiB segments where the parts are 16-byte aligned, the launch
+    touches more than 80 MB or the check copies the unit as well; with every part on whole cache lines also for 1 KiB
+    segments above 80 MB and, in the copying check, multiples of 512 bytes up to 4 KiB below; the chain loop otherwise."""
+    far = (2 if fused else 1) * sum(parts) > 80000000
+    if seg == 2048:
+        lds = fused or far or all(pb % 16 == 0 for pb in parts)
+    else:
+        lds = (seg == 1024 if far else fused and seg % 512 == 0 and seg <= 4096) and all(pb % 128 == 0 for pb in parts)
     if fused:
         return "dg_scatter_verify_lds_kernel" if lds else "dg_scatter_verify_kernel"
     return "dg_verify_lds_kernel" if lds else "dg_verify_kernel"
@@ -635,7 +640,7 @@ def main():
 
         copy_gbps = pprof["copy_bytes"] / pprof["copy_ns"] if pprof["copy_ns"] else None
         # units with a part under 8 MiB are staged, and with device verify their scatter is the check
-        # (dg_scatter_verify_kernel): each landed unit is read from HBM staging and written to its slot once
+        # (dg_scatter_verify_lds_kernel): each landed unit is read from HBM staging and written to its slot once
         fused = len(w.parts) > 1 and min(w.parts) < (8 << 20)
         ver_bytes = prof["verify_bytes"] * (2 if fused else 1)
         traffic_unit = (SCATTER_VERIFY_TRAFFIC_PER_UNIT if fused else VERIFY_TRAFFIC_PER_UNIT).get(w.unit_bytes)
@@ -884,14 +889,14 @@ def run_host(a, w, tsa, ss, W, L, C):
 
 
 def host_roofline(prof, w):
-    """The host contract's dominant kernel: verify_kernel, the device XXH64 of each batch of landed units (up to 32 per
+    """The host contract's dominant kernel: verify_lds_kernel, the device XXH64 of each batch of landed units (up to 32 per
     launch), live over the timed steps."""
     if not prof["verifies"] or not prof["verify_ns"]:
         return None
     gbps = prof["verify_bytes"] / prof["verify_ns"]
     per_launch = prof["verify_bytes"] / prof["verifies"]
     ratio = HOST_VERIFY_TRAFFIC_RATIO.get(w.unit_bytes)
-    return {"bound": "hbm", "kernel": "verify_kernel (device XXH64 of each batch of landed units)",
+    return {"bound": "hbm", "kernel": "verify_lds_kernel (device XXH64 of each batch of landed units)",
             "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(gbps / HBM_PEAK_GBPS, 4),
             "traffic": int(ratio * per_launch) if ratio else None,
             "traffic_source": HOST_TRAFFIC_SOURCE.get(w.unit_bytes),

@@ -84,7 +84,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 // Two normals of one source word by Box-Muller (below), as bf16 values, the cosine's in the low half.
 // The angle is exact up to its last step: lo32 counts 2^-32 turns, so its nearest quarter turn q and the signed rest r
 // (lo32 << 2 as a signed number, in 2^-34 turns) are integer work, and only r, within an eighth of a turn, is rounded.
-// sin and cos of the rest are polynomials in x^2 fitted here to |x| <= pi / 4 (relative error 3.6e-9 and 9.5e-11, both
+// sin and cos of the rest are polynomials in x^2 fitted here to |x| <= pi / 4 (relative error 6.1e-9 and 7.0e-10, both
 // under the 6e-8 of a 32-bit rounding). Logarithm and square root are the hardware's (1 ulp).
 __device__ __forceinline__ uint32_t normal_pair(uint64_t w, float sigma) {
   uint32_t hi = uint32_t(w >> 32);
@@ -111,7 +111,7 @@ __device__ __forceinline__ uint32_t normal_pair(uint64_t w, float sigma) {
 // u1 = (hi32 + 0.5) / 2^32, u2 = (lo32 + 0.5) / 2^32, r = sigma sqrt(-2 ln u1), (r cos 2 pi u2, r sin 2 pi u2); a
 // 64-bit output word then holds elements 4w .. 4w + 3, i.e. source words 2w and 2w + 1. A lane makes two output words
 // and stores them at once; the source words' counters step by kGolden, one product per lane. Kind 1 is bound by its
-// arithmetic, about 52 vector instructions per source word of which 21 mix it: 112 MiB in 40.9 us (71.8 with the
+// arithmetic, about 52 vector instructions per source word of which 21 mix it: 112 MiB in 39.8 us (66.2 with the
 // library's sinf, cosf, logf and sqrtf), 17 us of it the store; the values nearest to the 64-bit ones in all but 2.3e-5
 // of the cases (1.6e-4). Kind 0: 112 MiB in 19.1 us (20.8 with 8-byte stores).
 template <uint32_t kKind>

@@ -1,4 +1,4 @@
-// Device XXH64 (seed 0) for units already resident in HBM, two kernels:
+// Device XXH64 (seed 0) for units already resident in HBM, in two ways:
 //
 //  * digest: XXH64 keeps four dependent 64-bit chains per input, each chain a sequence of rotl(v + w*P2, 31)*P1 steps.
 //    There is no associative combine, so a unit's digest is bound by its chains: one wave runs only them, fed with the
@@ -202,9 +202,9 @@ __global__ __launch_bounds__(256) void digest_quads_kernel(const TsaUnit* __rest
 // is everything the chain's wave issues: here it is only the chain. With b = rotl(acc + w P2, 31), the accumulator is
 // b P1 and the next round is b' = rotl(b P1 + w' P2, 31): one v_mad_u64_u32 (the product's low half, w' P2 added on the
 // way), two v_mul_lo_u32, an add and two funnel shifts: 25 cycles measured for one wave, 30 with its LDS reads (61 with
-// the word's own product in the same wave). One 9 MiB unit: 11.6 -> 3.62 ms; 128 of them: 15.8 -> 3.66 ms. The products w P2 come from four other waves of the workgroup: they
-// read the units' bytes in 16-byte pieces (whole lines), multiply, and lay each chain's products next to each other in
-// LDS, so that the hashing wave takes two rounds with one ds_read_b128.
+// the word's own product in the same wave). One 9 MiB unit: 11.6 -> 3.62 ms; 128 of them: 15.8 -> 3.66 ms. The products
+// w P2 come from four other waves of the workgroup: they read the units' bytes in 16-byte pieces (whole lines), multiply,
+// and lay each chain's products next to each other in LDS, so that the hashing wave takes two rounds with one ds_read_b128.
 //
 // A workgroup hashes kG units (4 kG lanes of its first wave); kG is a power of two, 512 / kG stripes of each unit make a
 // chunk (16 KiB), and three chunk buffers go round: while chunk k is hashed, chunk k+1 is complete (the hashing wave
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(64 + kFeeders) void digest_fed_kernel(const TsaUnit
 // both costs in them they were the launch's last: 8 MB in 5.5 us instead of 6.3).
 //
 // What bounds it: reading, from about 50 MB on (336 MiB in 56.1 us on changing buffers, 6.4 TB/s); below, one launch and
-// four or five memory latencies (192 KiB 5.4 us, of which a launch of nothing takes 3.7).
+// four or five memory latencies (192 KiB 5.0-5.2 us, of which a launch of nothing takes 3.7).
 template <uint32_t kD>  // per wave: kD chunk buffers, and 64 bytes of checkpoints per quad behind them
 constexpr uint32_t wave_lds_bytes() {
   return kD * 4096 + 64 * 16;
@@ -1028,8 +1028,9 @@ int launch_digest(const TsaUnit* units_dev, uint32_t n, uint64_t* out_dev, hipSt
 //    the lines 53 MB in 4 KiB ones 20.5 / 16.7, in 1 KiB ones 14.7 / 13.2, in 2 KiB ones 14.1 / 14.6.
 //
 // Two buffers a wave; four for the copy above 80 MB and for checks above it whose parts lie off the cache lines; all of a
-// segment's chunks in flight for checks of units (batches) of up to 96 segments of 2 KiB. Reads go past the caches, stores (the copy's) through them. Measured in workgroups of four waves, us (in a loop on changing buffers / one
-// launch after other reads):
+// segment's chunks in flight for checks of units (batches) of up to 96 segments of 2 KiB. Reads go past the caches, stores
+// (the copy's) through them. Measured in workgroups of four waves, us (in a loop on changing buffers / one launch after
+// other reads):
 //  * Four buffers, 70 KB of LDS a workgroup, two on a CU. On whole lines: 85 MB 16.0 / 19.9, two 15.5 / 19.0; 358 MB 56.9 /
 //    58.8, two 56.4 / 59.5; 307 MB batch 48.8 / 53.4, two 47.9 / 51.0. Off them: 358 MB 62.6 / 65.0, two 71.4 / 73.9; 178 MB
 //    32.1 / 37.7, two 35.0 / 41.8 (a batch's extents are not known here: two). The copy: 150 MB moved 28.8 / 31.6, two 30.0 /
