@@ -77,10 +77,11 @@ def test_synth_edges(gpu, kind, words, offset):
             assert np.array_equal(got, synth.uniform_bytes(99, 5, at, n) if kind == 0 else synth.q4_blocks(99, 5, at, n))
 
 
-# The checks by segment size and by size: two chunk buffers a wave (2 KiB segments; on whole cache lines 1 KiB ones above 80
-# MB and, in the copy, any whole pair of 256-byte chunks up to 4 KiB and 80 MB, above 1 KiB), the chain loop (other
-# segments; up to 80 MB also arenas with a part that is 8-byte aligned; above, and in batches and the copy, the waves
-# that hold one); units in rows of workgroups or packed; parts that end inside a segment, inside a stripe, or are none.
+# The checks by segment size and by size. Streamed: 2 KiB segments; on whole cache lines also 1 KiB ones above 80 MB and, in
+# the copy, any whole pair of 256-byte chunks up to 4 KiB and 80 MB, above 1 KiB. Two chunk buffers a wave, four above 80 MB
+# in the copy and off the cache lines, all chunks in flight up to 96 segments of 2 KiB. The chain loop: other segments; up to
+# 80 MB also arenas with a part that is 8-byte aligned; above, and in batches and the copy, the waves that hold one. Units in
+# rows of workgroups or packed; parts that end inside a segment, inside a stripe, or are none.
 SHAPES = [
     (1, [2048], 2048), (1, [32], 2048), (2, [8], 2048), (1, [2080, 40], 2048), (5, [65568, 4096, 1000], 2048),
     (64, [30 * 2048 + 32, 96], 2048), (3, [2048 * 17, 2048 * 15 + 64, 32, 2048], 2048), (3, [(8 << 20) + 32, 1 << 20], 2048),
@@ -88,7 +89,8 @@ SHAPES = [
     (2, [9 << 20, 1024 * 3 + 8], 1024), (3, [1536 * 40 + 32, 1536 * 16 - 8], 1536), (2, [1 << 20, 4096 * 3 + 56], 4096), (2, [1 << 20, 4096 * 3 + 128], 4096),
     (1, [65536, 40], 4096), (2, [65536 + 64, 128], 1536), (64, [530016, 40], 2048), (70, [530016, 48], 2048),
     (3, [28 << 20, 4096 + 16], 4096), (3, [28 << 20, (3 << 20) + 1000], 1024),
-    (3, [44 << 20, (3 << 20) + 48], 1024), (2, [44 << 20, (3 << 20) + 128], 1024), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
+    (1, [84 << 20, (3 << 20) + 48], 2048),
+    (3, [32 * 2048, 64 * 2048], 2048), (3, [32 * 2048, 64 * 2048 + 64], 2048), (3, [44 << 20, (3 << 20) + 48], 1024), (2, [44 << 20, (3 << 20) + 128], 1024), (2, [1 << 20, 8192 + 32], 8192), (2, [1 << 18, 4000], 2080),
 ]
 
 

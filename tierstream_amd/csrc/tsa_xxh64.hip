@@ -1107,9 +1107,10 @@ int launch_dg_verify(const DgVerifyLaunch& a, hipStream_t stream, hipEvent_t sta
   const bool stream_it = check_streams(a.seg_bytes, bytes) &&
                          (aligned(a, stream_align(a.seg_bytes)) || (a.seg_bytes == 2048 && bytes > kNearBytes));
   const bool few = a.seg_bytes == 2048 && a.unit_segs <= kFewSegs;
+  static_assert(kDgVerifyMax * ((kFewSegs + 63) / 64) <= kCus, "a launch of few segments a unit is never packed");
   const bool four = stream_it && bytes > kNearBytes && !aligned(a, 128);
   auto* k = !stream_it ? (waves ? dev::dg_verify_kernel<true> : dev::dg_verify_kernel<false>)
-            : few      ? (waves ? dev::dg_verify_lds_kernel<8, true> : dev::dg_verify_lds_kernel<8, false>)
+            : few      ? dev::dg_verify_lds_kernel<8, false>
             : four     ? (waves ? dev::dg_verify_lds_kernel<4, true> : dev::dg_verify_lds_kernel<4, false>)
                        : (waves ? dev::dg_verify_lds_kernel<2, true> : dev::dg_verify_lds_kernel<2, false>);
   const int e = launch_timed(k, grid, 256, stream, start, stop, a, waves);
